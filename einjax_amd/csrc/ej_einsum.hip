@@ -10,6 +10,7 @@
 #include <ctype.h>
 #include <string.h>
 
+#include "ej_stream.h"
 #include "ej_internal.h"
 
 namespace ej {
@@ -228,100 +229,6 @@ namespace ej {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Shared pair addressing.
-
-struct PairSrc {
-  const int64_t *lidx, *ridx;  // null: identity
-  const int32_t *perm;         // null: identity
-  const int32_t *seg_off;      // null: one pair per segment
-  int64_t n_a_tiles, n_b_tiles;
-  const int64_t *n_live;       // non-null: segments >= *n_live are skipped (grid is a bound)
-  const int32_t *run_order;    // non-null: grouped launches run group run_order[b] as block b
-  int32_t order_group;         // segments per group that run_order was made for
-};
-
-// Whether the workgroup's segment lies beyond the device-side segment count.
-__device__ inline bool seg_dead(const PairSrc &s, int64_t seg) {
-  return s.n_live && seg >= *s.n_live;
-}
-
-__device__ inline void seg_range(const PairSrc &s, int64_t seg, int64_t *q0, int64_t *q1) {
-  if (s.seg_off) {
-    *q0 = s.seg_off[seg];
-    *q1 = s.seg_off[seg + 1];
-  } else {
-    *q0 = seg;
-    *q1 = seg + 1;
-  }
-}
-
-// Tiles of the q-th pair in plan order; false if an index is out of range.
-__device__ inline bool pair_tiles(const PairSrc &s, int64_t q, int64_t *at, int64_t *bt) {
-  int64_t p = s.perm ? s.perm[q] : q;
-  *at = s.lidx ? s.lidx[p] : p;
-  *bt = s.ridx ? s.ridx[p] : p;
-  return *at >= 0 && *at < s.n_a_tiles && *bt >= 0 && *bt < s.n_b_tiles;
-}
-
-__device__ inline float to_f32(float x) { return x; }
-__device__ inline float to_f32(uint16_t x) { return __uint_as_float(static_cast<uint32_t>(x) << 16); }
-
-// Output element stores: fp32 as is, bf16 rounded to nearest even
-// (v_cvt_pk_bf16_f32).  Sums are always formed in fp32; a bf16 output is
-// rounded once, when the finished tile is written.
-__device__ inline void put_out(float *p, float v) { *p = v; }
-__device__ inline void put_out(uint16_t *p, float v) {
-  *p = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
-}
-
-// Reads a workgroup-uniform element of a read-only index array through the
-// scalar cache, so the load does not occupy the vector memory counter that
-// paces the LDS ring.
-template <typename T>
-__device__ inline T ld_uniform(const T *p, int64_t i) {
-  return ((const __attribute__((address_space(4))) T *)(p))[i];
-}
-
-// Maps the first `live` block ids onto logical blocks (block id b runs on XCD
-// b % 8).  run == 0: the logical range is split into 8 contiguous parts, one
-// per XCD, so that neighbouring logical blocks (sharing operand tiles) share
-// an L2 over the widest window.  run > 0: runs of `run` consecutive logical
-// blocks go to one XCD, the runs dealt to the XCDs in turn, so that every XCD
-// gets a share of each region of the logical range (work that is heavier in
-// one region, as for skewed sparsity, stays balanced); the last, partial
-// round of runs is split into 8 contiguous parts.  Block ids from `live` on
-// keep their id: they lie beyond the work of a grid sized for a bound.
-__device__ inline int64_t xcd_logical_block(int64_t live, int64_t run = 0) {
-  const int64_t bid = blockIdx.x;
-  if (bid >= live) return bid;
-  const int64_t full = run > 0 ? live / (8 * run) * (8 * run) : 0;
-  const int64_t xcd = bid % 8;
-  if (bid < full) {
-    const int64_t local = bid / 8;
-    return ((local / run) * 8 + xcd) * run + local % run;
-  }
-  const int64_t rest = live - full, local = (bid - full) / 8;
-  const int64_t per = rest / 8, rem = rest % 8;
-  const int64_t start = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
-  return full + start + local;
-}
-
-// Run length of the dealt mapping for one-segment workgroups taken in plan
-// order (no run order): their neighbours share few tiles, and skewed
-// sparsity makes whole regions of the plan heavier.
-constexpr int64_t kXcdRun = 16;
-
-// Blocks that carry work when each segment takes blocks_per_seg of them: the
-// whole grid, or, given a device-side segment count, that many segments' blocks
-// (so that a grid sized for a bound still spreads its live work over every XCD).
-__device__ inline int64_t live_blocks(const PairSrc &s, int64_t blocks_per_seg) {
-  const int64_t total = gridDim.x;
-  if (!s.n_live) return total;
-  const int64_t live = ld_uniform(s.n_live, 0) * blocks_per_seg;
-  return live < total ? live : total;
-}
-
-// ---------------------------------------------------------------------------
 // MFMA grouped GEMM.
 //
 // One workgroup (4 waves, 2x2) computes a BM x BN block of one output tile
@@ -334,17 +241,6 @@ __device__ inline int64_t live_blocks(const PairSrc &s, int64_t blocks_per_seg) 
 // after them, so one barrier per stage suffices and HBM/L2 latency overlaps
 // the math.  The tile indices of the next pair are fetched one pair ahead.
 // Accumulation is fp32 in registers; each output block is written once.
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-struct GemmGeom {
-  int64_t m, n, k, batch;
-  int64_t a_sb, a_sm, a_sk, b_sb, b_sk, b_sn, c_sb, c_sm, c_sn;
-  int64_t a_elems, b_elems, c_elems;
-  int64_t mblocks, nblocks;
-  int32_t out_bf16;  // output tiles in bf16 (else fp32)
-};
 
 // LDS placement of a [rows][BK] operand chunk in 16-byte chunks of VEC
 // elements.  With 128-byte rows (8 chunks) the chunk index is XOR-swizzled
@@ -2083,6 +1979,36 @@ bool try_gemm(const ej_einsum_desc *d, int32_t dtype, const void *A, const void 
   return true;
 }
 
+// The streaming GEMM for the GEMM-shaped einsums that the blocked kernels do
+// not take (extents that are no multiples of their blocks, rows that are not
+// 16-byte aligned): any extents and strides with at least one lane's k values
+// per row, tiles of less than 2 GB and 31-bit tile indices.  K below that
+// (outer and elementwise products) stays with the generic kernel: a K block
+// would be nearly all padding.
+bool try_stream(const ej_einsum_desc *d, int32_t dtype, const void *A, const void *B, void *C,
+                const PairSrc &src, int64_t n_seg, hipStream_t stream, int *status) {
+  const int64_t esz = dtype == EJ_BF16 ? 2 : 4;
+  if (!d->is_gemm || d->k < 16 / esz) return false;
+  const int64_t lim = int64_t(1) << 31;
+  if (d->a_elems * esz >= lim || d->b_elems * esz >= lim || d->c_elems * 4 >= lim ||
+      src.n_a_tiles >= lim || src.n_b_tiles >= lim || n_seg >= lim)
+    return false;
+  if (n_seg * ceil_div(d->m, 16) * ceil_div(d->n, 16) * d->batch >= lim) return false;
+  const int am = d->a_sk == 1 ? kStreamKC : d->a_sm == 1 ? kStreamFC : kStreamGS;
+  const int bm = d->b_sk == 1 ? kStreamKC : d->b_sn == 1 ? kStreamFC : kStreamGS;
+  GemmGeom g;
+  g.m = d->m; g.n = d->n; g.k = d->k; g.batch = d->batch;
+  g.a_sb = d->a_sb; g.a_sm = d->a_sm; g.a_sk = d->a_sk;
+  g.b_sb = d->b_sb; g.b_sk = d->b_sk; g.b_sn = d->b_sn;
+  g.c_sb = d->c_sb; g.c_sm = d->c_sm; g.c_sn = d->c_sn;
+  g.a_elems = d->a_elems; g.b_elems = d->b_elems; g.c_elems = d->c_elems;
+  g.mblocks = g.nblocks = 1;
+  g.out_bf16 = d->out_dtype == EJ_BF16;
+  *status = dtype == EJ_BF16 ? launch_stream_bf16(am, bm, A, B, C, src, g, n_seg, stream)
+                             : launch_stream_f32(am, bm, A, B, C, src, g, n_seg, stream);
+  return true;
+}
+
 int run_generic(const ej_einsum_desc *d, int32_t dtype, const void *A, const void *B, void *C,
                 const PairSrc &src, int64_t n_seg, hipStream_t stream) {
   GenDesc g;
@@ -2199,6 +2125,7 @@ int einsum_common(const ej_einsum_desc *d, int32_t dtype, const void *A, const v
   EJ_TRY(check_desc(d));
   int status = EJ_OK;
   if (dtype != EJ_I32 && try_gemm(d, dtype, A, B, C, src, n_seg, stream, &status)) return status;
+  if (dtype != EJ_I32 && try_stream(d, dtype, A, B, C, src, n_seg, stream, &status)) return status;
   return run_generic(d, dtype, A, B, C, src, n_seg, stream);
 }
 

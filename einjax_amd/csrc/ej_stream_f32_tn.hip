@@ -1,0 +1,7 @@
+// Streaming tile GEMM on f32 tiles, the layout of one gradient of a matmul.
+#include "ej_stream.h"
+
+namespace ej {
+template int launch_stream_m<float, kStreamFC, kStreamFC>(
+    const void *, const void *, void *, const PairSrc &, const GemmGeom &, int64_t, hipStream_t);
+}  // namespace ej

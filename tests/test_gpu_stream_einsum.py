@@ -1,0 +1,122 @@
+"""Tile einsums on extents the blocked MFMA kernels do not take (the streaming
+GEMM): every number of 16-wide fragments and its edges, K tails, all operand
+layouts, one and four waves per output block, against float64."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import reference_path as R
+
+from einjax_amd import _device
+
+pytestmark = pytest.mark.gpu
+
+# m, k, n: fragment edges (16), block edges (5 fragments), K blocks of 16 (fp32)
+# and 32 (bf16) with their tails, single rows and columns, several blocks.
+SIZES = [(1, 8, 1), (16, 16, 16), (17, 15, 33), (33, 31, 17), (48, 33, 49), (75, 75, 75),
+         (80, 80, 81), (81, 47, 80), (5, 100, 64), (64, 9, 1), (100, 20, 125), (161, 24, 97)]
+SPECS = {"ij,jk->ik": ("mk", "kn"), "ij,kj->ik": ("mk", "nk"), "ji,jk->ik": ("km", "kn"),
+         "ji,kj->ik": ("km", "nk"), "ij,jk->ki": ("mk", "kn")}
+
+
+def _tol(dtype, out, products):
+    """rel-L2 bound: every product and partial sum rounds to 2^-24 of its
+    value, which over a sum of n terms grows as sqrt(n); a bf16 result (8
+    significand bits) rounds once more, by at most 2^-8 of itself."""
+    return 2.0 ** -24 * np.sqrt(products) * 2 + (2.0 ** -8 if out == torch.bfloat16 else 0)
+
+
+def _case(spec, m, k, n, dtype, seed, tiles=7, pairs=40, segs=9):
+    rng = np.random.default_rng(seed)
+    ext = dict(m=m, k=k, n=n)
+    lt, rt = (tuple(ext[x] for x in t) for t in SPECS[spec])
+    lv, rv = (rng.standard_normal((tiles, *t)).astype(np.float32) for t in (lt, rt))
+    if dtype == torch.bfloat16:
+        lv, rv = R.bf16_round(lv), R.bf16_round(rv)
+    li, ri = rng.integers(0, tiles, pairs), rng.integers(0, tiles, pairs)
+    off = np.sort(np.concatenate([[0, pairs], rng.integers(0, pairs, segs - 1)])).astype(np.int32)
+    perm = rng.permutation(pairs).astype(np.int32)
+    return lt, rt, lv, rv, li, ri, perm, off
+
+
+def _run(spec, lt, rt, lv, rv, li, ri, perm, off, dtype, out=None):
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    return _device.segment_einsum(_device.describe(spec, lt, rt), dev(lv).to(dtype),
+                                  dev(rv).to(dtype), dev(li), dev(ri), dev(perm), dev(off), out)
+
+
+@pytest.mark.parametrize("spec", SPECS)
+@pytest.mark.parametrize("m,k,n", SIZES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_segments(gpu, spec, m, k, n, dtype):
+    """Segments of zero to many pairs: few blocks, four waves each."""
+    print("[case] stream segments", spec, m, k, n, dtype, flush=True)
+    c = _case(spec, m, k, n, dtype, m * 131 + k * 17 + n)
+    lt, rt, lv, rv, li, ri, perm, off = c
+    pv = R.kernel_einsum(lv, rv, li, ri, spec, precision="fp64")[perm]
+    want = np.stack([pv[a:b].sum(0) for a, b in zip(off[:-1], off[1:])])
+    longest = int(np.diff(off).max()) * k
+    for out in {dtype, torch.float32}:
+        got = _run(spec, *c, dtype, out)
+        assert got.dtype == out
+        err = R.rel_l2(got.float().cpu().numpy(), want)
+        assert err <= _tol(dtype, out, longest), (out, err)
+    empty = np.flatnonzero(np.diff(off) == 0)
+    assert not got[torch.from_numpy(empty).cuda()].any()
+
+
+@pytest.mark.parametrize("m,k,n,spec", [(20, 20, 20, "ij,jk->ik"), (75, 75, 75, "ij,jk->ik"),
+                                        (36, 25, 50, "ij,kj->ik"), (50, 45, 33, "ji,jk->ik")])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_many_pairs_one_wave_each(gpu, m, k, n, spec, dtype):
+    """Per-pair results of more pairs than split blocks, and of a few of them
+    (four waves): within rounding of float64, and the two splits of each other."""
+    print("[case] stream pairs", spec, m, k, n, dtype, flush=True)
+    lt, rt, lv, rv, li, ri, _, _ = _case(spec, m, k, n, dtype, 3, pairs=2500)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    desc = _device.describe(spec, lt, rt)
+    args = dev(lv).to(dtype), dev(rv).to(dtype)
+    many = _device.pair_einsum(desc, *args, dev(li), dev(ri))
+    few = _device.pair_einsum(desc, *args, dev(li[:300]), dev(ri[:300]))
+    want = R.kernel_einsum(lv, rv, li, ri, spec, precision="fp64")
+    for got, ref in ((many, want), (few, want[:300])):
+        assert R.rel_l2(got.float().cpu().numpy(), ref) <= _tol(dtype, dtype, k)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("spec", ["ij,jk->ik", "ij,kj->ik", "ji,jk->ik", "ji,kj->ik"])
+def test_neighbour_tiles_and_invalid_pairs(gpu, spec, dtype):
+    """A K tail or an edge never mixes in the neighbouring tiles (all NaN
+    here), and a pair with an index out of range adds nothing."""
+    print("[case] stream neighbours", spec, dtype, flush=True)
+    m, k, n = 35, 21, 50
+    lt, rt, lv, rv, _, _, _, _ = _case(spec, m, k, n, dtype, 11)
+    lv[[0, 2]] = np.nan
+    rv[[0, 2]] = np.nan
+    li, ri = np.array([1, 1, 9, 1, -1]), np.array([1, 1, 1, 9, 1])
+    off, perm = np.array([0, 1, 5], np.int32), np.arange(5, dtype=np.int32)
+    got = _run(spec, lt, rt, lv, rv, li, ri, perm, off, dtype, torch.float32).cpu().numpy()
+    want = R.kernel_einsum(lv, rv, li[:1], ri[:1], spec, precision="fp64")[0]
+    assert R.rel_l2(got[0], want) <= _tol(dtype, torch.float32, k)
+    np.testing.assert_array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_unaligned_base_and_batch(gpu, dtype):
+    """Tiles at an address that is no multiple of 16, and a batch label."""
+    print("[case] stream unaligned", dtype, flush=True)
+    rng = np.random.default_rng(2)
+    spec, lt, rt = "bij,bjk->bik", (3, 19, 37), (3, 37, 21)
+    lv, rv = (R.bf16_round(rng.standard_normal((5, *t)).astype(np.float32)) for t in (lt, rt))
+    li, ri = rng.integers(0, 5, 30), rng.integers(0, 5, 30)
+
+    def shifted(a):
+        flat = torch.zeros(a.size + 1, dtype=dtype, device="cuda")
+        flat[1:] = torch.from_numpy(a.reshape(-1)).cuda().to(dtype)
+        return flat[1:].view(a.shape)
+
+    got = _device.pair_einsum(_device.describe(spec, lt, rt), shifted(lv), shifted(rv),
+                              torch.from_numpy(li).cuda(), torch.from_numpy(ri).cuda())
+    want = R.kernel_einsum(lv, rv, li, ri, spec, precision="fp64")
+    assert R.rel_l2(got.float().cpu().numpy(), want) <= _tol(dtype, dtype, 37)
