@@ -477,3 +477,34 @@ def test_row_step_answers_changed_data(gpu):
                             precision="fp64")
     npt.assert_array_equal(got.coords.cpu().numpy(), want.coords)
     assert R.rel_l2(got.values.cpu().numpy(), want.values) <= 1e-5
+
+
+@pytest.mark.parametrize("shape,density,other", [
+    ((1, 1), 1.0, 1.0), ((7, 73), 1.0, 0.5), ((16, 32), 1.0, 1.0), ((27, 19), 1.0, 0.02),
+    ((40, 30), 0.4, 0.3), ((3, 20, 30), 0.5, 0.4), ((128, 64), 1.0, 0.7), ((90, 90), 0.9, 0.9)])
+def test_row_plan_tile_with_tile(gpu, shape, density, other):
+    """Joins on every dim (elementwise products): 1, 511, 512 and 513 lhs
+    tiles (one block of 512 and its neighbours) up to the plan's 8,192 runs,
+    few and all of them matched; then one pair too many for either capacity,
+    bad data, and a good call after it."""
+    note("row plan tile with tile", shape, density, other)
+    rng = np.random.default_rng(len(shape) + shape[0])
+    L, Rr = (rel_from_mask(rng, rng.random(shape) < d) for d in (density, other))
+    Rr.coords[0] = L.coords[-1] if len(Rr.coords) == 1 else Rr.coords[0]  # at least one match
+    keys = [(d, d) for d in range(len(shape))]
+    agg = [(0, d) for d in range(len(shape))]
+    li_o, uc, segs = oracle_segments(L, Rr, keys, agg)
+    P = len(li_o)
+    for direct in (False, True):
+        st, res = run_row(L, Rr, keys, agg, cap_p=max(P, 1), direct=direct)
+        assert st == _lib.EJ_OK and res["counts"] == [P, 0, P, 0, P, 0]
+        npt.assert_array_equal(res["coords"], uc)
+        npt.assert_array_equal(res["off"], np.arange(P + 1))
+        npt.assert_array_equal(res["li"], [s[0][0] for s in segs])
+        npt.assert_array_equal(res["ri"], [s[1][0] for s in segs])
+    if P > 1:
+        assert run_row(L, Rr, keys, agg, cap_p=P - 1, cap_u=P)[1]["counts"] == [0, 2, P - 1, 0, P, 0]
+        assert run_row(L, Rr, keys, agg, cap_p=P, cap_u=P - 1)[1]["counts"] == [0, 2, P, 0, P, 0]
+        bad = R.Rel(L.coords[::-1].copy(), L.values, L.shape, L.tile_shape)
+        assert run_row(bad, Rr, keys, agg, cap_p=P)[1]["counts"][:2] == [0, 1]
+        assert run_row(L, Rr, keys, agg, cap_p=P)[1]["counts"][:2] == [P, 0]
