@@ -508,3 +508,48 @@ def test_row_plan_tile_with_tile(gpu, shape, density, other):
         bad = R.Rel(L.coords[::-1].copy(), L.values, L.shape, L.tile_shape)
         assert run_row(bad, Rr, keys, agg, cap_p=P)[1]["counts"][:2] == [0, 1]
         assert run_row(L, Rr, keys, agg, cap_p=P)[1]["counts"][:2] == [P, 0]
+
+
+@pytest.mark.parametrize("tile", [(1,), (3, 5), (64, 64), (25, 41), (129, 33)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32])
+def test_elementwise_tiles(gpu, tile, dtype):
+    """Elementwise tile products summed over segments of 0 to several pairs:
+    one element, partial vectors, several 16 KB workgroups, tiles off 16-byte
+    alignment; integers exactly, bf16 as its fp32 result rounded."""
+    note("elementwise tiles", tile, dtype)
+    rng = np.random.default_rng(sum(tile))
+    lab = "ij"[:len(tile)]
+    spec = f"{lab},{lab}->{lab}"
+    n, P = 6, 14
+    if dtype == torch.int32:
+        lv, rv = (torch.from_numpy(rng.integers(-2**31, 2**31, (n, *tile)).astype(np.int32)).cuda()
+                  for _ in range(2))
+    else:
+        lv, rv = (torch.from_numpy(rng.standard_normal((n, *tile)).astype(np.float32)).cuda()
+                  .to(dtype) for _ in range(2))
+    li, ri = rng.integers(0, n, P), rng.integers(0, n, P)
+    li[3] = n  # out of range: adds nothing
+    off = np.array([0, 1, 1, 5, P], np.int32)
+    perm = rng.permutation(P).astype(np.int32)
+    dev = lambda a: torch.from_numpy(a).cuda()
+    desc = _device.describe(spec, tile, tile)
+    args = (lv, rv, dev(li), dev(ri), dev(perm), dev(off))
+    got = _device.segment_einsum(desc, *args)
+    if dtype == torch.int32:
+        a, b = (v.cpu().numpy().astype(np.int64) for v in (lv, rv))
+    else:
+        a, b = (v.double().cpu().numpy() for v in (lv, rv))
+    want = np.zeros((4, *tile), a.dtype)
+    for u in range(4):
+        for q in perm[off[u]:off[u + 1]]:
+            if li[q] < n:
+                want[u] += a[li[q]] * b[ri[q]] if dtype != torch.int32 else (
+                    (a[li[q]] * b[ri[q]]) & 0xFFFFFFFF)
+    if dtype == torch.int32:
+        npt.assert_array_equal(got.cpu().numpy(), want.astype(np.uint32).view(np.int32))
+        return
+    f32 = got if dtype == torch.float32 else _device.segment_einsum(desc, *args, torch.float32)
+    # nine products at most: each product and each sum rounds to 2^-24 of itself
+    assert R.rel_l2(f32.cpu().numpy(), want) <= 10 * 2.0 ** -24
+    if dtype == torch.bfloat16:
+        assert torch.equal(got, f32.to(torch.bfloat16))
