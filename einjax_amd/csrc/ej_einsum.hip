@@ -391,15 +391,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 3 : 2) void tile_gemm_kernel(
   __shared__ __align__(16) T As[2][BM * LDK];
   __shared__ __align__(16) T Bs[2][BN * LDK];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  int64_t lb = xcd_logical_block(live_blocks(src, g.nblocks * g.mblocks * g.batch));
-  const int64_t nb = lb % g.nblocks;
-  lb /= g.nblocks;
-  const int64_t mb = lb % g.mblocks;
-  lb /= g.mblocks;
-  const int64_t bi = lb % g.batch;
-  const int64_t seg = lb / g.batch;
+  const BlockPos pos =
+      block_pos(xcd_logical_block(live_blocks(src, g.nblocks * g.mblocks * g.batch)), g);
+  const int64_t nb = pos.nb, mb = pos.mb, bi = pos.bi, seg = pos.seg;
   if (seg_dead(src, seg)) return;
 
   int64_t q0, q1;
@@ -665,15 +662,12 @@ __global__ __launch_bounds__(256) void tile_gemm_dma_kernel(const uint16_t *__re
   const uint32_t ring_lds = static_cast<uint32_t>(
       reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char *)ring));
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  int64_t lb = xcd_logical_block(live_blocks(src, g.nblocks * g.mblocks * g.batch));
-  const int64_t nb = lb % g.nblocks;
-  lb /= g.nblocks;
-  const int64_t mb = lb % g.mblocks;
-  lb /= g.mblocks;
-  const int64_t bi = lb % g.batch;
-  const int64_t seg = lb / g.batch;
+  const BlockPos pos =
+      block_pos(xcd_logical_block(live_blocks(src, g.nblocks * g.mblocks * g.batch)), g);
+  const int64_t nb = pos.nb, mb = pos.mb, bi = pos.bi, seg = pos.seg;
   if (seg_dead(src, seg)) return;
   int64_t q0, q1;
   seg_range(src, seg, &q0, &q1);
@@ -1152,7 +1146,8 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
   const uint32_t ring_lds = static_cast<uint32_t>(
       reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char *)ring));
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
   const int wseg = (wn * WN) / BN;  // segment (inside a group) of this wave's columns
   const int wcol = (wn * WN) % BN;  // its first column inside that segment's tile
@@ -1160,25 +1155,20 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
   // [seg0, seg0 + nls) for one n-block and one batch index.
   const int segs = G > 1 || !MULTI ? G : spw;
   int64_t nseg = n_seg;
-  int64_t live = gridDim.x;  // blocks with work
+  uint32_t live = gridDim.x;  // blocks with work
   if (src.n_live) {
     const int64_t nl = ld_uniform(src.n_live, 0);
     nseg = nl < nseg ? nl : nseg;
     const int64_t per_grp = g.nblocks * (MULTI && mb_loop ? 1 : g.mblocks) * g.batch;
-    const int64_t lg = (nseg + segs - 1) / segs * per_grp;
-    live = lg < live ? lg : live;
+    // segs is a power of two
+    const int64_t lg = ((nseg + segs - 1) >> (31 - __builtin_clz(segs))) * per_grp;
+    live = lg < live ? static_cast<uint32_t>(lg) : live;
   }
-  int64_t lb = xcd_logical_block(live, G == 1 && !src.run_order ? kXcdRun : 0);
-  const int64_t nb = lb % g.nblocks;
-  lb /= g.nblocks;
-  int64_t mb0 = 0, nmb = g.mblocks;
-  if (!MULTI || !mb_loop) {
-    mb0 = lb % g.mblocks;
-    lb /= g.mblocks;
-    nmb = 1;
-  }
-  const int64_t bi = lb % g.batch;
-  int64_t grp = lb / g.batch;
+  const bool all_m = MULTI && mb_loop;
+  const BlockPos pos =
+      block_pos(xcd_logical_block(live, G == 1 && !src.run_order ? kXcdRun : 0), g, all_m);
+  const int64_t nb = pos.nb, mb0 = pos.mb, nmb = all_m ? g.mblocks : 1, bi = pos.bi;
+  int64_t grp = pos.seg;
   if (grp * segs >= nseg) return;
   // A run order (for instance heaviest groups first on each XCD) replaces
   // the block's group (its n-, m- and batch blocks stay together).  Its header, run_order[0], is the number of live groups it
@@ -1187,7 +1177,7 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
   // every block alike, so each live group runs once; any other order is
   // ignored as a whole.
   if (!MULTI && src.run_order) {
-    const int64_t ngroups = (nseg + segs - 1) / segs;
+    const int64_t ngroups = (nseg + G - 1) / G;  // segs == G
     if (ld_uniform(src.run_order, 0) == ngroups) {
       const int64_t o = ld_uniform(src.run_order, grp + 1);
       if (o >= 0 && o < ngroups) grp = o;
@@ -1298,8 +1288,9 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
   // Issue cursor: m-block imb, pair ipos, K-chunk ikc.
   int64_t imb = mb0, ipos = 0;
   int ikc = 0;
+  int islot = 0;       // ring slot of the next stage to issue
   uint64_t codes = 0;  // 8 bits per ring slot
-  auto issue = [&](int64_t st) {
+  auto issue = [&]() {
     if ((ipos >> 6) != chunk) {  // more than 64 pairs per m-block only
       if (uni) load_shared(static_cast<int>(ipos >> 6));
       else load_seq(static_cast<int>(ipos >> 6));
@@ -1319,7 +1310,7 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
       code = static_cast<uint32_t>(lane_value(tsg, li)) | (at < 0 ? kSkip : 0u);
     }
     const int64_t a_tile = at < 0 ? 0 : at;
-    unsigned char *slot = ring + (st % NS) * SLOT;
+    unsigned char *slot = ring + islot * SLOT;
     const TA *ab = A + a_tile * g.a_elems + bi * g.a_sb + imb * BM * g.a_sm + ikc * BK * g.a_sk;
 #pragma unroll
     for (int v = 0; v < LPA; ++v)
@@ -1335,8 +1326,9 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
             bb + b_src[v], EJ_LDS(slot + A_BYTES + s * B_BYTES + (v * NW + wave) * 1024), 16, 0,
             0);
     }
-    const int sh = static_cast<int>(st % NS) * 8;
+    const int sh = islot * 8;
     codes = (codes & ~(uint64_t(0xFF) << sh)) | (uint64_t(code) << sh);
+    islot = islot + 1 == NS ? 0 : islot + 1;
     if (++ikc == nkc) {
       ikc = 0;
       if (++ipos == npos) {
@@ -1376,15 +1368,17 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
 
 #pragma unroll
   for (int s0 = 0; s0 < NS - 1; ++s0)
-    if (s0 < stages) issue(s0);
+    if (s0 < stages) issue();
 
   uint32_t rd[Op::template n_rd<FM, FN>];
   Op::template read_offsets<FM, FN>(rd, wm * WM, wcol,
                                     static_cast<uint32_t>(A_BYTES + wseg * B_BYTES), lane);
   int64_t cmb = mb0;      // compute cursor's m-block
   int64_t cleft = per_mb;  // stages left in it
+  int next_slot = 0;
   for (int64_t st = 0; st < stages; ++st) {
-    const int slot = static_cast<int>(st % NS);
+    const int slot = next_slot;
+    next_slot = slot + 1 == NS ? 0 : slot + 1;
     // The next stage goes into the slot of stage st - 1 as soon as every
     // wave is done with it, before this stage's data is waited for, so NS - 1
     // stages are in flight while the waves wait and NS - 2 while they compute.
@@ -1392,7 +1386,7 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
     }
-    if (st + NS - 1 < stages) issue(st + NS - 1);
+    if (st + NS - 1 < stages) issue();
     const int64_t later = stages - 1 - st < NS - 1 ? stages - 1 - st : NS - 1;
     wait_stage_in<NS, LPS>(static_cast<int>(later));
     __builtin_amdgcn_s_barrier();
@@ -1553,7 +1547,7 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
     bool done = --cleft == 0;
     if constexpr (G == 1) {
       if (!done && !uni) {
-        const uint32_t nxt = static_cast<uint32_t>(codes >> (((st + 1) % NS) * 8)) & 0xFu;
+        const uint32_t nxt = static_cast<uint32_t>(codes >> (next_slot * 8)) & 0xFu;
         done = nxt != (code & 0xFu);
       }
     }

@@ -70,34 +70,48 @@ __device__ inline T ld_uniform(const T *p, int64_t i) {
 // one region, as for skewed sparsity, stays balanced); the last, partial
 // round of runs is split into 8 contiguous parts.  Block ids from `live` on
 // keep their id: they lie beyond the work of a grid sized for a bound.
-__device__ inline int64_t xcd_logical_block(int64_t live, int64_t run = 0) {
-  const int64_t bid = blockIdx.x;
+__device__ inline uint32_t xcd_logical_block(uint32_t live, uint32_t run = 0) {
+  const uint32_t bid = blockIdx.x;
   if (bid >= live) return bid;
-  const int64_t full = run > 0 ? live / (8 * run) * (8 * run) : 0;
-  const int64_t xcd = bid % 8;
+  const uint32_t full = run > 0 ? live / (8 * run) * (8 * run) : 0;
+  const uint32_t xcd = bid % 8;
   if (bid < full) {
-    const int64_t local = bid / 8;
+    const uint32_t local = bid / 8;
     return ((local / run) * 8 + xcd) * run + local % run;
   }
-  const int64_t rest = live - full, local = (bid - full) / 8;
-  const int64_t per = rest / 8, rem = rest % 8;
-  const int64_t start = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
+  const uint32_t rest = live - full, local = (bid - full) / 8;
+  const uint32_t per = rest / 8, rem = rest % 8;
+  const uint32_t start = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
   return full + start + local;
+}
+
+// x / d (and the remainder) of workgroup-uniform values, kept in scalar
+// registers.  A division runs on the vector unit (a 64-bit one takes over a
+// hundred instructions), and what follows from its result would stay there:
+// one division of 1 is the common case and costs nothing.
+__device__ inline uint32_t div_uniform(uint32_t x, uint32_t d, uint32_t *rem) {
+  if (d == 1) {
+    *rem = 0;
+    return x;
+  }
+  const uint32_t q = __builtin_amdgcn_readfirstlane(x / d);
+  *rem = x - q * d;
+  return q;
 }
 
 // Run length of the dealt mapping for one-segment workgroups taken in plan
 // order (no run order): their neighbours share few tiles, and skewed
 // sparsity makes whole regions of the plan heavier.
-constexpr int64_t kXcdRun = 16;
+constexpr uint32_t kXcdRun = 16;
 
 // Blocks that carry work when each segment takes blocks_per_seg of them: the
 // whole grid, or, given a device-side segment count, that many segments' blocks
 // (so that a grid sized for a bound still spreads its live work over every XCD).
-__device__ inline int64_t live_blocks(const PairSrc &s, int64_t blocks_per_seg) {
-  const int64_t total = gridDim.x;
+__device__ inline uint32_t live_blocks(const PairSrc &s, int64_t blocks_per_seg) {
+  const uint32_t total = gridDim.x;
   if (!s.n_live) return total;
   const int64_t live = ld_uniform(s.n_live, 0) * blocks_per_seg;
-  return live < total ? live : total;
+  return live < total ? static_cast<uint32_t>(live) : total;
 }
 
 // ---------------------------------------------------------------------------
@@ -113,5 +127,18 @@ struct GemmGeom {
   int64_t mblocks, nblocks;
   int32_t out_bf16;  // output tiles in bf16 (else fp32)
 };
+
+// Where an output block lies: n-block, m-block, batch index, segment (or
+// group of segments) of logical block lb.
+struct BlockPos {
+  uint32_t nb, mb, bi, seg;
+};
+__device__ inline BlockPos block_pos(uint32_t lb, const GemmGeom &g, bool all_m = false) {
+  BlockPos p{0, 0, 0, 0};
+  lb = div_uniform(lb, static_cast<uint32_t>(g.nblocks), &p.nb);
+  if (!all_m) lb = div_uniform(lb, static_cast<uint32_t>(g.mblocks), &p.mb);
+  p.seg = div_uniform(lb, static_cast<uint32_t>(g.batch), &p.bi);
+  return p;
+}
 
 }  // namespace ej

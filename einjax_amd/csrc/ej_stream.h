@@ -283,17 +283,14 @@ __global__ __launch_bounds__(256, stream_waves(FM * FN)) void stream_gemm_kernel
     nseg = nl < nseg ? nl : nseg;
   }
   constexpr int UPB = 4 / W;  // output blocks per workgroup
-  const int64_t units = nseg * per_seg;
-  const int64_t live = (units + UPB - 1) / UPB;
-  if (static_cast<int64_t>(blockIdx.x) >= live) return;
-  int64_t lb = xcd_logical_block(live, kXcdRun) * UPB + (W == 1 ? wave : 0);
+  const uint32_t units = static_cast<uint32_t>(nseg * per_seg);  // below 2^31 (launch_stream_t)
+  const uint32_t live = (units + UPB - 1) / UPB;
+  if (blockIdx.x >= live) return;
+  const uint32_t lb = xcd_logical_block(live, kXcdRun) * UPB + (W == 1 ? wave : 0);
   if (lb >= units) return;  // W = 1 only: no barrier follows
-  const int nb = static_cast<int>(lb % g.nblocks);
-  lb /= g.nblocks;
-  const int mb = static_cast<int>(lb % g.mblocks);
-  lb /= g.mblocks;
-  const int64_t bi = lb % g.batch;
-  const int64_t seg = lb / g.batch;
+  const BlockPos at_block = block_pos(lb, g);
+  const int nb = static_cast<int>(at_block.nb), mb = static_cast<int>(at_block.mb);
+  const int64_t bi = at_block.bi, seg = at_block.seg;
   const int32_t q0 = src.seg_off ? ld_uniform(src.seg_off, seg) : static_cast<int32_t>(seg);
   const int32_t q1 = src.seg_off ? ld_uniform(src.seg_off, seg + 1) : q0 + 1;
   const int M = static_cast<int>(g.m), N = static_cast<int>(g.n), K = static_cast<int>(g.k);
