@@ -1114,7 +1114,7 @@ struct SegOpSplitB {
   }
 };
 
-template <class Op, int NS, int G, int WGM, int NW, bool MULTI>
+template <class Op, int NS, int G, int WGM, int NW, bool MULTI, bool LINES>
 __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op::a_elem *__restrict__ A,
                                                            const typename Op::b_elem *__restrict__ B,
                                                            void *__restrict__ C, PairSrc src,
@@ -1353,6 +1353,37 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
   auto block_off = [&](int sseg, int64_t mb) -> int64_t {  // in elements
     return (seg0 + sseg) * g.c_elems + bi * g.c_sb + mb * BM * g.c_sm + nb * BN * g.c_sn;
   };
+  // LINES: a bf16 block with 16-byte rows leaves in whole lines of WN columns.
+  // 64 lanes' worth of rows at a time goes through a strip of LDS of the
+  // wave's own (rows of 8 bytes more than the data, so that the rows of a
+  // write fall on different banks) and is stored 16 bytes a lane.
+  constexpr int LPR = WN * 2 / 16;            // lanes per row
+  constexpr int LR = LPR >= 8 ? 2 : 4;        // result rows of a lane per step
+  constexpr int LROW = WN * 2 + 8;            // bytes per strip row
+  static_assert(!LINES || LPR * 4 * LR == 64, "a step fills the wave");
+  __shared__ __align__(16) unsigned char strip[LINES ? NW * 4 * LR * LROW : 16];
+  auto store_lines = [&](uint16_t *cb, int64_t csm) {  // cb: the wave's first element
+    unsigned char *st = strip + wave * (4 * LR * LROW);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int r0 = 0; r0 < 4; r0 += LR) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int r = 0; r < LR; ++r)
+            put_out(reinterpret_cast<uint16_t *>(st + ((lane >> 4) * LR + r) * LROW) + j * 16 +
+                        (lane & 15), acc[i][j][r0 + r]);
+        const int x = lane / LPR, ch = lane % LPR;
+        const uint2 lo = *reinterpret_cast<const uint2 *>(st + x * LROW + ch * 16);
+        const uint2 hi = *reinterpret_cast<const uint2 *>(st + x * LROW + ch * 16 + 8);
+        const int row = i * 16 + x / LR * 4 + r0 + x % LR;
+        *reinterpret_cast<uint4 *>(cb + row * csm + ch * 8) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      }
+  };
+  const bool lines = LINES && g.out_bf16 && g.c_sn == 1 &&
+                     ((g.c_sm | g.c_sb | g.c_elems) & 7) == 0 &&
+                     (reinterpret_cast<size_t>(C) & 15u) == 0;
   auto store_zero = [&](int sseg, int64_t mb) {
     if (sseg >= nls) return;
     auto zero = [&](auto *cb) {
@@ -1569,7 +1600,8 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
                 put_out(cb + o0 + (i * 16 + r) * csm + j * 16 * csn, acc[i][j][r]);
         };
         const int64_t c0 = block_off(sseg, cmb);
-        if (g.out_bf16) store(static_cast<uint16_t *>(C) + c0);
+        if (lines) store_lines(static_cast<uint16_t *>(C) + c0 + (wm * WM) * csm + wcol, csm);
+        else if (g.out_bf16) store(static_cast<uint16_t *>(C) + c0);
         else store(static_cast<float *>(C) + c0);
       }
 #pragma unroll
@@ -1597,7 +1629,8 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
             }
       };
       const int64_t c0 = block_off(wseg, mb0);
-      if (g.out_bf16) store(static_cast<uint16_t *>(C) + c0);
+      if (lines) store_lines(static_cast<uint16_t *>(C) + c0 + (wm * WM) * g.c_sm + wcol, g.c_sm);
+      else if (g.out_bf16) store(static_cast<uint16_t *>(C) + c0);
       else store(static_cast<float *>(C) + c0);
     }
     return;
@@ -1881,7 +1914,7 @@ SegSplit seg_split(int G, int64_t n_seg, int64_t batch, int64_t nblocks, int64_t
   return r;
 }
 
-template <class Op, int G, int WGM, int NW, int NSW = EJ_SEG_NS>
+template <class Op, int G, int WGM, int NW, int NSW = EJ_SEG_NS, bool LINES = false>
 int launch_seg_gemm_t(const void *A, const void *B, void *C, const PairSrc &src_in,
                       const GemmGeom &g, int64_t n_seg, hipStream_t stream) {
   constexpr int NS = seg_ring_depth(Op::A_BYTES + G * Op::B_BYTES, NSW);
@@ -1899,12 +1932,12 @@ int launch_seg_gemm_t(const void *A, const void *B, void *C, const PairSrc &src_
   using TA = typename Op::a_elem;
   using TB = typename Op::b_elem;
   if (mb_loop || spw > 1)
-    hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, true>),
+    hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, true, LINES>),
                        dim3(static_cast<unsigned>(nblk)), dim3(NW * 64), 0, stream,
                        static_cast<const TA *>(A), static_cast<const TB *>(B), C, src, g, n_seg,
                        spw, mb_loop);
   else
-    hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, false>),
+    hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, false, LINES>),
                        dim3(static_cast<unsigned>(nblk)), dim3(NW * 64), 0, stream,
                        static_cast<const TA *>(A), static_cast<const TB *>(B), C, src, g, n_seg, 1,
                        0);
@@ -2037,6 +2070,22 @@ bool try_gemm(const ej_einsum_desc *d, int32_t dtype, const void *A, const void 
     const uint16_t *a = static_cast<const uint16_t *>(A);
     const uint16_t *b = static_cast<const uint16_t *>(B);
     const bool grouped = src.seg_off && d->seg_group > 0 && d->seg_group % 4 == 0;
+    // Per-pair results (no segment sums): the ring kernel with 32-deep stages
+    // and whole-line stores. Its 37 KB of LDS let four workgroups share a CU,
+    // so that one's loads run under another's stores, most of the traffic
+    // here (26,208 pairs of 128 x 128 x 128: 859 MB written; empty workgroups
+    // alone take 51 us, stores alone 121, loads and MFMAs alone 178). Measured
+    // against tile_gemm_dma_kernel: those pairs 303 / 357 us, 13,107 pairs of
+    // 64 x 64 x 64 42 / 71 us. With segments the two are within 10% of each
+    // other either way, so those keep the 64-deep kernel below.
+    if (!src.seg_off && ad && !bd) {
+      *status = bm == 128
+                    ? launch_seg_gemm_t<SegOpBf16<128, 128>, 1, 2, 4, EJ_SEG_NS, true>(
+                          A, B, C, src, g, n_seg, stream)
+                    : launch_seg_gemm_t<SegOpBf16<64, 64>, 1, 2, 4, EJ_SEG_NS, true>(
+                          A, B, C, src, g, n_seg, stream);
+      return true;
+    }
     if (grouped || d->k % 64 != 0 || !ad || bd) {
       *status = launch_seg_gemm_bf16(bm, grouped ? 4 : 1, ad, bd, a, b, C, src, g, n_seg, stream);
       return true;

@@ -120,3 +120,33 @@ def test_unaligned_base_and_batch(gpu, dtype):
                               torch.from_numpy(li).cuda(), torch.from_numpy(ri).cuda())
     want = R.kernel_einsum(lv, rv, li, ri, spec, precision="fp64")
     assert R.rel_l2(got.float().cpu().numpy(), want) <= _tol(dtype, dtype, 37)
+
+
+@pytest.mark.parametrize("m,k,n", [(64, 32, 64), (64, 96, 192), (128, 32, 128), (256, 64, 128),
+                                   (128, 160, 256)])
+@pytest.mark.parametrize("spec", ["ij,jk->ik", "ij,jk->ki"])
+def test_pair_results_in_lines(gpu, m, k, n, spec):
+    """Per-pair bf16 results of 64 and 128 blocks: rows stored in lines (bf16
+    results), as they come (fp32 results, transposed results, an output that is
+    not 16-byte aligned): all of them one fp32 result, rounded once."""
+    print("[case] pair lines", spec, m, k, n, flush=True)
+    from einjax_amd import _lib
+    import ctypes
+
+    lt, rt, lv, rv, li, ri, _, _ = _case("ij,jk->ik", m, k, n, torch.bfloat16, m + k + n)
+    li[3] = len(lv)  # out of range: a tile of zeros
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    a, b, dli, dri = dev(lv).bfloat16(), dev(rv).bfloat16(), dev(li), dev(ri)
+    desc = _device.describe(spec, lt, rt)
+    f32 = _device.pair_einsum(desc, a, b, dli, dri, out_dtype=torch.float32)
+    got = _device.pair_einsum(desc, a, b, dli, dri)
+    want = R.kernel_einsum(lv, rv, np.where(li < len(lv), li, 0), ri, spec, precision="fp64")
+    want[3] = 0
+    assert R.rel_l2(f32.cpu().numpy(), want) <= _tol(torch.bfloat16, torch.float32, k)
+    assert torch.equal(got, f32.bfloat16())
+    flat = torch.zeros(got.numel() + 1, dtype=torch.bfloat16, device="cuda")
+    assert _lib.load().ej_pair_einsum(
+        ctypes.byref(desc), _lib.EJ_BF16, _device.ptr(a), _device.ptr(b), a.shape[0], b.shape[0],
+        _device.ptr(dli), _device.ptr(dri), len(li), _device.ptr(flat[1:]),
+        _device.stream_ptr()) == _lib.EJ_OK
+    assert torch.equal(flat[1:].view(got.shape), got)
