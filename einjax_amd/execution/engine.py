@@ -144,7 +144,8 @@ class ExecutionEngine:
             raise NotImplementedError("dense einsum steps are not part of einjax_amd; the "
                                       "engine runs steps whose operands are SparseTensorRelation")
         join, agg = relation_einsum_plan(formula, lhs.tile_shape, rhs.tile_shape)
-        return execute_sparse(lhs, rhs, join, formula, agg, **self.step_options)
+        return execute_sparse(lhs, rhs, join, formula, agg,
+                              **{"_new_relations": True, **self.step_options})
 
     def execute_plan(self, plan, operands: list, gather_output: bool = False):
         """Runs plan.steps in order over a working list that starts as the

@@ -460,6 +460,38 @@ def _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound, pair_key,
     return None
 
 
+# Output buffers of a guessed step hold at most this (larger einsums are not
+# bound by the waits the guess saves).
+_GUESS_MAX_BYTES = 256 << 20
+
+
+def _pair_guess(lhs, rhs, keys, kernel_string, nl: int, nr: int, out_dtype):
+    """A pair bound for the first call on two relations, for callers that seldom
+    make a second one, so that it too can queue the row plan and the einsum
+    without waiting for a count: the pairs of uniformly spread tiles and a
+    quarter more.  A guess that is too small
+    is detected on the device and costs one more plan with the exact count.
+    None where the general plan is to answer: large outputs, a stream under
+    capture (the count's wait would not end), or a call the library would
+    refuse only once there are pairs.
+    A three-operand chain on 32 x 32 fp32 tiles, whose second step always
+    meets a new relation: 302 us a call with the general plan and its
+    host waits, 179-188 us so."""
+    import torch
+
+    if out_dtype not in (None, torch.float32) or torch.cuda.is_current_stream_capturing():
+        return None
+    cells = 1
+    for _, d in keys:
+        cells *= _grid(rhs, d)
+    guess = int(1.25 * nl * nr / max(cells, 1)) + 64
+    try:
+        elems = _device.describe(kernel_string, lhs.tile_shape, rhs.tile_shape).c_elems
+    except (ValueError, TypeError, RuntimeError):
+        return None
+    return guess if 4 * elems * guess <= _GUESS_MAX_BYTES else None
+
+
 # ---------------------------------------------------------------------------
 # Repeated calls.  A queued step on device relations keeps its prepared plan
 # and einsum (a DenseStep or QueuedStep: argument lists, capacities, output
@@ -776,11 +808,11 @@ def _empty_result(lhs, n_out, out_tile, output_shape, host, out_dtype=None):
 def execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_keys,
                    kernel_string: str, agg_keys, output_shape=None, output_tile_shape=None, *,
                    fused: bool = True, out_dtype=None,
-                   _einsum_events=None) -> SparseTensorRelation:
+                   _einsum_events=None, _new_relations: bool = False) -> SparseTensorRelation:
     try:
         return _execute_sparse(lhs, rhs, join_keys, kernel_string, agg_keys, output_shape,
                                output_tile_shape, fused=fused, out_dtype=out_dtype,
-                               _einsum_events=_einsum_events)
+                               _einsum_events=_einsum_events, _new_relations=_new_relations)
     except _NegativeCoords:
         pass
     # Negative joined or output coordinates: run on columns shifted to be
@@ -813,7 +845,7 @@ def execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_ke
 def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_keys,
                     kernel_string: str, agg_keys, output_shape=None, output_tile_shape=None, *,
                     fused: bool = True, out_dtype=None,
-                    _einsum_events=None) -> SparseTensorRelation:
+                    _einsum_events=None, _new_relations: bool = False) -> SparseTensorRelation:
     """Sparse tensor-relational einsum (reference: sparse_dispatch.py:226-297).
 
     join_keys: [(lhs_dim, rhs_dim)] contracted tile dims; kernel_string: the
@@ -828,7 +860,9 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
     for bfloat16 tiles, rounded once from the fp32 sum); ``torch.float32``
     keeps fp32 results for bfloat16 tiles.  ``_einsum_events`` (measurement
     only): a list that collects timing events recorded around the fused
-    einsum of a queued call.  Integer or boolean tiles (and a float with an
+    einsum of a queued call.  ``_new_relations`` (the engine's steps): the
+    relations are made anew for each call, so a first call is queued on a
+    guessed pair bound (_pair_guess).  Integer or boolean tiles (and a float with an
     integer) follow the reference's jnp promotion (kernel_einsum) and run on
     the library's integer kernel; joined and output coordinates may be
     negative."""
@@ -893,7 +927,7 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
     keys = [tuple(k) for k in join_keys]
     hint_key = None
     bound = None
-    queued = None
+    queued = guess = None
     if fused and keys and lc.shape[0] and rc.shape[0] and not integer:
         done = _dense_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, _einsum_events)
         if done is not None:
@@ -906,9 +940,12 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
         hint_key = _hint_key(lhs, rhs, (tuple(lc.shape), tuple(rc.shape), tuple(keys),
                                         tuple(j_rad), tuple(agg)))
         bound = _hint_get(hint_key, lhs, rhs)
-        if bound is not None and bound > 0:
-            done = _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound, hint_key,
-                             _einsum_events)
+        if bound is None and _new_relations:
+            guess = _pair_guess(lhs, rhs, keys, kernel_string, lc.shape[0], rc.shape[0],
+                                out_dtype)
+        if (bound or guess or 0) > 0:
+            done = _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound or guess,
+                             hint_key, _einsum_events)
             if done is not None:
                 queued, step, rkey = done
                 kind, dkey = "row", (hint_key, rkey)
@@ -928,7 +965,8 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
     if queued is not None:
         P, U, coords, vals, _ = queued
         step.result_tile, step.result_shape = output_tile_shape, output_shape
-        if (step_key is not None and not host and tuple(step.out_tile) == output_tile_shape
+        # (a step with guessed capacities is not kept: the next call has the count)
+        if (step_key is not None and guess is None and not host and tuple(step.out_tile) == output_tile_shape
                 and step.n_out == n_out):
             _remember_step(step_key, lhs, rhs, kind, step, dkey, fin)
         if P == 0:

@@ -553,3 +553,43 @@ def test_elementwise_tiles(gpu, tile, dtype):
     assert R.rel_l2(f32.cpu().numpy(), want) <= 10 * 2.0 ** -24
     if dtype == torch.bfloat16:
         assert torch.equal(got, f32.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("case", ["uniform", "skewed", "empty", "unsorted"])
+def test_first_call_queues_row_plan(gpu, case, monkeypatch):
+    """The first call on relations made anew takes a guessed pair bound: enough, too
+    small (one rerun with the count), no pairs at all, or data the row plan
+    does not take; the result is bitwise the general plan's."""
+    note("first call", case)
+    rng = np.random.default_rng(7)
+    a, b = sparse_rel(rng, (24, 40), (32, 32), 0.2), sparse_rel(rng, (40, 16), (32, 32), 0.2)
+    if case == "skewed":  # every tile on one join index
+        ca = np.stack([np.arange(24), np.full(24, 3)], axis=1).astype(np.int32)
+        cb = np.stack([np.full(16, 3), np.arange(16)], axis=1).astype(np.int32)
+        a = R.Rel(ca, a.values[:24], a.shape, a.tile_shape)
+        b = R.Rel(cb, b.values[:16], b.shape, b.tile_shape)
+    elif case == "empty":
+        ka, kb = a.coords[:, 1] == 0, b.coords[:, 0] > 0
+        a = R.Rel(a.coords[ka], a.values[ka], a.shape, a.tile_shape)
+        b = R.Rel(b.coords[kb], b.values[kb], b.shape, b.tile_shape)
+    L, Rr = dev_rel(a), dev_rel(b)
+    if case == "unsorted":
+        p = torch.from_numpy(rng.permutation(len(a.coords))).cuda()
+        L = SparseTensorRelation(L.coords[p].contiguous(), L.values[p].contiguous(), a.shape,
+                                 a.tile_shape)
+    statuses = []
+    run = _device.run_row_step
+
+    def spy(step, events=None):
+        r = run(step, events)
+        statuses.append(r[0])
+        return r
+
+    monkeypatch.setattr(_device, "run_row_step", spy)
+    args = ([(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)])
+    got = ej.execute_sparse(L, Rr, *args, _new_relations=True)
+    assert statuses == {"uniform": ["ok"], "skewed": ["bound", "ok"], "empty": ["ok"],
+                        "unsorted": ["miss"]}[case]
+    sd._pair_hints.clear()
+    want = ej.execute_sparse(L, Rr, *args)
+    assert torch.equal(got.coords, want.coords) and torch.equal(got.values, want.values)
