@@ -331,3 +331,44 @@ def test_scheme_stats_order3_all_tile_shapes(gpu):
     assert D.count_nonzero(dense) == len(coords) * 32 ** 3
     del dense
     torch.cuda.empty_cache()
+
+
+# ---------------------------------------------------------------------------
+# tiles by vectors: rows that are whole 16-byte vectors, rows whose last vector
+# overlaps, rows below one vector (element kernels), several vectors a thread
+
+@pytest.mark.parametrize("dtype", ["f64", "f32", "bf16"])
+@pytest.mark.parametrize("grid,tile", [((3, 5), (128, 128)), ((4, 3), (25, 75)), ((2, 3), (7, 8)),
+                                       ((5, 2), (130, 9)), ((3, 4), (6, 1)), ((2, 2, 3), (5, 3, 11)),
+                                       ((3,), (17,)), ((2, 2), (3, 300)), ((1, 2), (96, 250))])
+def test_dense_tiles_round_trip(gpu, dtype, grid, tile):
+    note("dense tiles round trip", dtype, grid, tile)
+    rng = np.random.default_rng(prod(tile))
+    shape = tuple(g * t for g, t in zip(grid, tile))
+    keep = rng.random(grid) < 0.5
+    keep.flat[0] = True
+    d = rng.standard_normal(shape)
+    mask = keep
+    for ax, t in enumerate(tile):
+        mask = np.repeat(mask, t, axis=ax)
+    d = np.where(mask, d, -0.0)
+    d.flat[0] = np.nan
+    # a tile whose only nonzero element is its last one
+    last = tuple(slice((g - 1) * t, g * t) for g, t in zip(grid, tile))
+    d[last] = 0.0
+    d[tuple(s - 1 for s in shape)] = 5e-324 if dtype == "f64" else 1.5
+    dev, exact = to_device(d, dtype)
+    buf = torch.empty(dev.numel() + 1, dtype=dev.dtype, device="cuda")
+    for x in (dev, buf[1:].view(shape).copy_(dev)):  # aligned, and off by one element
+        rel = SparseTensor("A", x).to_relation(tile)
+        blocks = exact.reshape([v for g, t in zip(grid, tile) for v in (g, t)])
+        nd = len(grid)
+        blocks = blocks.transpose([2 * i for i in range(nd)] + [2 * i + 1 for i in range(nd)])
+        has = (blocks != 0).reshape(*grid, -1).any(axis=-1)
+        coords = np.argwhere(has)
+        npt.assert_array_equal(rel.coords.cpu().numpy(), coords)
+        got = rel.values.double().cpu().numpy()
+        want = blocks[tuple(coords.T)]
+        npt.assert_array_equal(got, want)
+        assert not np.signbit(got[got == 0]).any()  # zeros are stored as +0.0
+        npt.assert_array_equal(rel.to_dense().double().cpu().numpy(), exact)
