@@ -80,16 +80,34 @@ __device__ inline int wave_incl_i32(int v) {
   return v;
 }
 
-// Adds the block's total of v to *acc: one atomic per 256-thread block.
-// Every thread of the block calls it.
+// Sum over the wave in lane 63, by DPP moves as wave_inclusive_sum.
+template <int CTRL, int ROWS>
+__device__ inline uint32_t dpp_add(uint32_t v) {
+  return v + static_cast<uint32_t>(
+                 __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xf, false));
+}
+__device__ inline uint32_t wave_total_u32(uint32_t v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15, 31
+  return dpp_add<0x143, 0xc>(v);
+}
+
+// Adds the block's total of v to *acc: one atomic per NT-thread block.  Every
+// thread of the block calls it.  (Atomics on one address take 12 ns each, one
+// after the other: kernels that read at full rate take few, large blocks.)
+template <int NT = 256>
 __device__ inline void block_add(unsigned long long *acc, int64_t v) {
-  __shared__ int64_t part[4];
+  __shared__ int64_t part[NT / 64];
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
-    const int64_t t = part[0] + part[1] + part[2] + part[3];
+    int64_t t = 0;
+    for (int w = 0; w < NT / 64; ++w) t += part[w];
     if (t) atomicAdd(acc, static_cast<unsigned long long>(t));
   }
 }
@@ -609,54 +627,97 @@ struct TileIdx {  // mixed-radix tile index of an element for one tile shape
 // 32-bit words (bit i of the map is bit i % 32 of word i / 32); bits past the
 // last tile are zero.
 
+// Flag bits of a 16-byte vector: bit k = element k is nonzero.  bf16: adding
+// 0x7fff to a half's magnitude carries into its top bit exactly when it is not
+// zero, and never out of the half; even elements end at even bits and odd ones
+// 15 above them.
+__device__ inline uint32_t nz_bits(const uint16_t *, uint4 x) {
+  auto z = [](uint32_t w) { return ((w & 0x7fff7fffu) + 0x7fff7fffu) & 0x80008000u; };
+  const uint32_t a = z(x.x) >> 15 | z(x.y) >> 13 | z(x.z) >> 11 | z(x.w) >> 9;
+  return (a | a >> 15) & 0xffu;
+}
+__device__ inline uint32_t nz_bits(const float *, uint4 x) {
+  auto z = [](uint32_t w) { return ((w & 0x7fffffffu) + 0x7fffffffu) >> 31; };
+  return z(x.x) | z(x.y) << 1 | z(x.z) << 2 | z(x.w) << 3;
+}
+__device__ inline uint32_t nz_bits(const double *, uint4 x) {
+  return ((x.x | (x.y & 0x7fffffffu)) != 0u ? 1u : 0u) |
+         ((x.z | (x.w & 0x7fffffffu)) != 0u ? 2u : 0u);
+}
+
+// v or-ed over aligned groups of N lanes (4, 8 or 16) by DPP moves.
+template <int CTRL>
+__device__ inline uint32_t dpp_or(uint32_t v) {
+  return v | static_cast<uint32_t>(
+                 __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xf, 0xf, true));
+}
+template <int N>
+__device__ inline uint32_t or_lanes(uint32_t v) {
+  static_assert(N == 4 || N == 8 || N == 16, "lanes per group");
+  v = dpp_or<0xB1>(v);                           // quad_perm 1, 0, 3, 2
+  v = dpp_or<0x4E>(v);                           // quad_perm 2, 3, 0, 1
+  if constexpr (N >= 8) v = dpp_or<0x141>(v);    // row_half_mirror
+  if constexpr (N >= 16) v = dpp_or<0x140>(v);   // row_mirror
+  return v;
+}
+
+// The map of a dense tensor: bound by its one read.  Each wave takes chunks
+// of 4 rounds x 64 lanes x 16 bytes (consecutive lanes read consecutive
+// bytes); the flag bits of the LPW lanes of a map word are or-ed by DPP moves,
+// and one store writes the four rounds' words (lane r of each group that of
+// round r).  512 blocks of 16 waves fill the chip: 8,192 blocks of four spent
+// much of the time on the count's atomics (16384^2 bf16: 135 us against 107 with
+// blocks of 1,024 threads; 162 / 150 us right after another 0.5 GB was written).
+constexpr int kBitsThreads = 1024, kBitsBlocks = 512;
+
 template <typename T>
-__global__ __launch_bounds__(256) void dense_bits_kernel(const T *__restrict__ dense, int64_t n,
+__global__ __launch_bounds__(kBitsThreads) void dense_bits_kernel(const T *__restrict__ dense, int64_t n,
                                                          bool vec, uint32_t *__restrict__ map,
                                                          unsigned long long *count) {
-  // Each wave takes chunks of 4 rounds x 64 lanes x E elements, one 16-byte
-  // load per lane and round (consecutive lanes read consecutive bytes); the
-  // E flag bits of LPW neighbouring lanes are or-ed into one map word by
-  // shuffles and stored by the first of them.
   constexpr int E = 16 / static_cast<int>(sizeof(T));  // elements per load
-  constexpr int LPW = 32 / E;                           // lanes per map word
+  constexpr int LPW = 32 / E;                          // lanes per map word
   constexpr int R = 4;
+  static_assert(R <= LPW, "one lane per round stores a word");
   constexpr int64_t CHUNK = int64_t(R) * 64 * E;
   const int lane = threadIdx.x & 63;
+  const int sub = lane % LPW;
   const int64_t words = (n + 31) / 32;
   const int64_t chunks = (n + CHUNK - 1) / CHUNK;
-  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * 4;
+  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * (kBitsThreads / 64);
   int64_t c = 0;
-  for (int64_t ch = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6); ch < chunks;
-       ch += n_waves) {
+  for (int64_t ch = static_cast<int64_t>(blockIdx.x) * (kBitsThreads / 64) + (threadIdx.x >> 6);
+       ch < chunks; ch += n_waves) {
     const int64_t base = ch * CHUNK;
-    T v[R][E];
+    uint4 v[R];
+    if (vec && base + CHUNK <= n) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int64_t i = base + static_cast<int64_t>(r * 64 + lane) * E;
-      if (vec && i + E <= n) {
-        const uint4 x = *reinterpret_cast<const uint4 *>(dense + i);
-        __builtin_memcpy(&v[r][0], &x, 16);
-      } else {
+      for (int r = 0; r < R; ++r)
+        v[r] = *reinterpret_cast<const uint4 *>(dense + base + (r * 64 + lane) * E);
+    } else {
 #pragma unroll
-        for (int k = 0; k < E; ++k) v[r][k] = i + k < n ? dense[i + k] : T(0);
+      for (int r = 0; r < R; ++r) {
+        T e[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+          const int64_t i = base + (r * 64 + lane) * E + k;
+          e[k] = i < n ? dense[i] : T(0);
+        }
+        __builtin_memcpy(&v[r], e, 16);
       }
     }
+    uint32_t w = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      uint32_t b = 0;
-#pragma unroll
-      for (int k = 0; k < E; ++k) b |= (nz(v[r][k]) ? 1u : 0u) << k;
-      b <<= E * (lane % LPW);
-#pragma unroll
-      for (int d = 1; d < LPW; d <<= 1) b |= __shfl_xor(b, d, 64);
-      const int64_t widx = (base + static_cast<int64_t>(r * 64 + lane) * E) >> 5;
-      if (lane % LPW == 0 && widx < words) {
-        map[widx] = b;
-        c += __popc(b);
-      }
+      const uint32_t b = or_lanes<LPW>(nz_bits(dense, v[r]) << (E * sub));
+      w = sub == r ? b : w;
+    }
+    const int64_t widx = (base >> 5) + sub * (64 / LPW) + lane / LPW;
+    if (sub < R && widx < words) {
+      map[widx] = w;
+      c += __popc(w);
     }
   }
-  block_add(count, c);
+  block_add<kBitsThreads>(count, c);
 }
 
 // Pooling by OR: in [outer][n_out * p][inner] -> out [outer][n_out][inner],
@@ -779,6 +840,38 @@ __device__ inline uint64_t level_mask(int k) {
   }
 }
 
+// Nonempty groups of 2^k bits, k = 1 .. 8, of a lane's 256 bits: add(k, count).
+// The eight 32-bit words are folded together: once pairs are or-ed, the free
+// odd bits of one word take the flags of the next, and so on at each level, so
+// that half as many words go on to the next one and the flags of all eight
+// meet in one byte (60 operations instead of the 200 of folding each
+// word).  Returns whether any bit is set.
+template <class Add>
+__device__ inline bool chain_levels(const uint64_t (&m)[4], Add add) {
+  uint32_t a[4], b[2];
+  auto fold = [](uint32_t x, int s, uint32_t mask) { return (x | x >> s) & mask; };
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    a[i] = fold(static_cast<uint32_t>(m[i]), 1, 0x55555555u) |
+           fold(static_cast<uint32_t>(m[i] >> 32), 1, 0x55555555u) << 1;
+  add(1, __popc(a[0]) + __popc(a[1]) + __popc(a[2]) + __popc(a[3]));
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    b[i] = fold(a[2 * i], 2, 0x33333333u) | fold(a[2 * i + 1], 2, 0x33333333u) << 2;
+  add(2, __popc(b[0]) + __popc(b[1]));
+  const uint32_t c = fold(b[0], 4, 0x0f0f0f0fu) | fold(b[1], 4, 0x0f0f0f0fu) << 4;
+  add(3, __popc(c));
+  const uint32_t d = fold(c, 8, 0x00ff00ffu);
+  add(4, __popc(d));
+  const uint32_t f = fold(d, 16, 0xffu);  // bit i: word i nonempty
+  add(5, __popc(f));
+  const uint32_t g6 = fold(f, 1, 0x55u);
+  add(6, __popc(g6));
+  add(7, __popc(fold(g6, 2, 0x11u)));
+  add(8, f != 0 ? 1 : 0);
+  return f != 0;
+}
+
 __global__ __launch_bounds__(256) void pool_chain_kernel(const uint32_t *__restrict__ in,
                                                          int64_t S, ChainArgs a,
                                                          uint32_t *__restrict__ out) {
@@ -809,21 +902,7 @@ __global__ __launch_bounds__(256) void pool_chain_kernel(const uint32_t *__restr
         }
       }
     }
-    uint64_t g[4] = {m[0], m[1], m[2], m[3]};
-#pragma unroll
-    for (int k = 1; k <= 6; ++k) {
-      int c = 0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        g[r] = (g[r] | (g[r] >> (1 << (k - 1)))) & level_mask(k);
-        c += __popcll(g[r]);
-      }
-      cnt[k - 1] += c;
-    }
-    // g[r] now holds bit 0 = word r nonempty
-    cnt[6] += (g[0] | g[1]) + (g[2] | g[3]);
-    const bool any = (g[0] | g[1] | g[2] | g[3]) != 0;
-    cnt[7] += any ? 1 : 0;
+    const bool any = chain_levels(m, [&](int k, int c) { cnt[k - 1] += c; });
     const uint64_t B = __ballot(any);
     uint64_t gb = B;
 #pragma unroll
@@ -862,9 +941,13 @@ __global__ __launch_bounds__(256) void pool_chain_kernel(const uint32_t *__restr
 // bits of every pooled row for k = 1 .. levels[h] as pool_chain_kernel does
 // (and, for h >= 1, the pooled map's own bits), and writes only the level-H
 // row.  Level 0's chain is counted when `first` is set (its map's own bits
-// were counted by its producer).  Counts: per lane, then one atomic per
-// counter and block.
+// were counted by its producer).  Counts: per lane, summed over the wave by
+// DPP moves (LDS-routed shuffles took 6 us of a launch), then one atomic per
+// counter and block.  The five launches of a 16384 x 16384 map take 47 us,
+// 89 us with shuffles and every word folded apart; the smallest are bound by
+// the latency of their one or two waves.
 constexpr int kBandMax = 3;  // row levels per launch: bands of 8 rows
+constexpr int kBandThreads = 256, kBandWaves = kBandThreads / 64;  // one atomic per counter and block
 
 struct BandArgs {
   int32_t H, first;
@@ -874,7 +957,7 @@ struct BandArgs {
   unsigned long long *pop[kBandMax + 1];
 };
 
-__global__ __launch_bounds__(256) void band_chain_kernel(const uint32_t *__restrict__ in,
+__global__ __launch_bounds__(kBandThreads) void band_chain_kernel(const uint32_t *__restrict__ in,
                                                          BandArgs a, uint32_t *__restrict__ out) {
   constexpr int NR = 1 << kBandMax;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -888,20 +971,7 @@ __global__ __launch_bounds__(256) void band_chain_kernel(const uint32_t *__restr
     for (int k = 0; k <= kChainMax; ++k) cnt[h][k] = 0;
   auto count = [&](const uint64_t (&m)[4], int h) {
     cnt[h][0] += __popcll(m[0]) + __popcll(m[1]) + __popcll(m[2]) + __popcll(m[3]);
-    uint64_t g[4] = {m[0], m[1], m[2], m[3]};
-#pragma unroll
-    for (int k = 1; k <= 6; ++k) {
-      uint32_t c = 0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        g[r] = (g[r] | (g[r] >> (1 << (k - 1)))) & level_mask(k);
-        c += __popcll(g[r]);
-      }
-      cnt[h][k] += c;
-    }
-    cnt[h][7] += static_cast<uint32_t>((g[0] | g[1]) + (g[2] | g[3]));
-    const bool any = (g[0] | g[1] | g[2] | g[3]) != 0;
-    cnt[h][8] += any ? 1u : 0u;
+    const bool any = chain_levels(m, [&](int k, int c) { cnt[h][k] += c; });
     uint64_t gb = __ballot(any);
 #pragma unroll
     for (int k = 9; k <= 14; ++k) {
@@ -909,8 +979,8 @@ __global__ __launch_bounds__(256) void band_chain_kernel(const uint32_t *__restr
       if (lane == 0) cnt[h][k] += __popcll(gb);
     }
   };
-  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * 4;
-  for (int64_t it = static_cast<int64_t>(blockIdx.x) * 4 + wave; it < items; it += n_waves) {
+  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kBandWaves;
+  for (int64_t it = static_cast<int64_t>(blockIdx.x) * kBandWaves + wave; it < items; it += n_waves) {
     const int64_t band = it / cpr, c = it - band * cpr;
     uint64_t m[NR][4];
 #pragma unroll
@@ -950,26 +1020,28 @@ __global__ __launch_bounds__(256) void band_chain_kernel(const uint32_t *__restr
                         static_cast<uint32_t>(m[0][3]), static_cast<uint32_t>(m[0][3] >> 32));
   }
   // Block totals: bits and levels 1-8 summed over the lanes, 9-14 held by lane 0.
-  __shared__ unsigned long long part[4][kBandMax + 1][kChainMax + 1];
+  __shared__ uint32_t part[kBandWaves][kBandMax + 1][kChainMax + 1];
 #pragma unroll
   for (int h = 0; h <= kBandMax; ++h)
 #pragma unroll
     for (int k = 0; k <= kChainMax; ++k) {
-      unsigned long long v = cnt[h][k];
+      if (h > H) continue;
       if (k <= 8) {
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+        const uint32_t v = wave_total_u32(cnt[h][k]);
+        if (lane == 63) part[wave][h][k] = v;
+      } else if (lane == 0) {
+        part[wave][h][k] = cnt[h][k];
       }
-      if (lane == 0) part[wave][h][k] = v;
     }
   __syncthreads();
-  for (int e = threadIdx.x; e < (kBandMax + 1) * (kChainMax + 1); e += 256) {
+  for (int e = threadIdx.x; e < (kBandMax + 1) * (kChainMax + 1); e += kBandThreads) {
     const int h = e / (kChainMax + 1), k = e % (kChainMax + 1);
     if (h > H) continue;
     unsigned long long *dst = nullptr;
     if (k == 0) dst = h >= 1 ? a.pop[h] : nullptr;
     else if (k <= a.levels[h] && (h >= 1 || a.first)) dst = a.chain[h][k - 1];
-    const unsigned long long t = part[0][h][k] + part[1][h][k] + part[2][h][k] + part[3][h][k];
+    unsigned long long t = 0;
+    for (int w = 0; w < kBandWaves; ++w) t += part[w][h][k];
     if (dst && t) atomicAdd(dst, t);
   }
 }
@@ -980,7 +1052,7 @@ __global__ __launch_bounds__(256) void band_chain_kernel(const uint32_t *__restr
 // many rows form a band inside it.  Level h ors each lane with the lane
 // lpr 2^(h-1) away (every lane of a group of 2^h rows then holds the group's
 // or); the first row's lanes of each group count it, the others are masked.
-__global__ __launch_bounds__(256) void band_chain_small_kernel(const uint32_t *__restrict__ in,
+__global__ __launch_bounds__(kBandThreads) void band_chain_small_kernel(const uint32_t *__restrict__ in,
                                                                BandArgs a,
                                                                uint32_t *__restrict__ out) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -998,19 +1070,7 @@ __global__ __launch_bounds__(256) void band_chain_small_kernel(const uint32_t *_
 #pragma unroll
     for (int r = 0; r < 4; ++r) g[r] = live ? m[r] : 0;
     cnt[h][0] += __popcll(g[0]) + __popcll(g[1]) + __popcll(g[2]) + __popcll(g[3]);
-#pragma unroll
-    for (int k = 1; k <= 6; ++k) {
-      uint32_t c = 0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        g[r] = (g[r] | (g[r] >> (1 << (k - 1)))) & level_mask(k);
-        c += __popcll(g[r]);
-      }
-      cnt[h][k] += c;
-    }
-    cnt[h][7] += static_cast<uint32_t>((g[0] | g[1]) + (g[2] | g[3]));
-    const bool any = (g[0] | g[1] | g[2] | g[3]) != 0;
-    cnt[h][8] += any ? 1u : 0u;
+    const bool any = chain_levels(g, [&](int k, int c) { cnt[h][k] += c; });
     uint64_t gb = __ballot(any);
 #pragma unroll
     for (int k = 9; k <= 14; ++k) {
@@ -1023,8 +1083,8 @@ __global__ __launch_bounds__(256) void band_chain_small_kernel(const uint32_t *_
     const uint32_t hi = __shfl_xor(static_cast<uint32_t>(v >> 32), d, 64);
     return static_cast<uint64_t>(lo) | static_cast<uint64_t>(hi) << 32;
   };
-  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * 4;
-  for (int64_t ch = static_cast<int64_t>(blockIdx.x) * 4 + wave; ch < chunks; ch += n_waves) {
+  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kBandWaves;
+  for (int64_t ch = static_cast<int64_t>(blockIdx.x) * kBandWaves + wave; ch < chunks; ch += n_waves) {
     const uint4 *src = reinterpret_cast<const uint4 *>(in) + (ch * kChainChunk + lane * 256) / 128;
     const uint4 v0 = src[0], v1 = src[1];
     uint64_t m[4];
@@ -1051,26 +1111,28 @@ __global__ __launch_bounds__(256) void band_chain_small_kernel(const uint32_t *_
                           static_cast<uint32_t>(m[3]), static_cast<uint32_t>(m[3] >> 32));
     }
   }
-  __shared__ unsigned long long part[4][kBandMax + 1][kChainMax + 1];
+  __shared__ uint32_t part[kBandWaves][kBandMax + 1][kChainMax + 1];
 #pragma unroll
   for (int h = 0; h <= kBandMax; ++h)
 #pragma unroll
     for (int k = 0; k <= kChainMax; ++k) {
-      unsigned long long v = cnt[h][k];
+      if (h > H) continue;
       if (k <= 8) {
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+        const uint32_t v = wave_total_u32(cnt[h][k]);
+        if (lane == 63) part[wave][h][k] = v;
+      } else if (lane == 0) {
+        part[wave][h][k] = cnt[h][k];
       }
-      if (lane == 0) part[wave][h][k] = v;
     }
   __syncthreads();
-  for (int e = threadIdx.x; e < (kBandMax + 1) * (kChainMax + 1); e += 256) {
+  for (int e = threadIdx.x; e < (kBandMax + 1) * (kChainMax + 1); e += kBandThreads) {
     const int h = e / (kChainMax + 1), k = e % (kChainMax + 1);
     if (h > H) continue;
     unsigned long long *dst = nullptr;
     if (k == 0) dst = h >= 1 ? a.pop[h] : nullptr;
     else if (k <= a.levels[h] && (h >= 1 || a.first)) dst = a.chain[h][k - 1];
-    const unsigned long long t = part[0][h][k] + part[1][h][k] + part[2][h][k] + part[3][h][k];
+    unsigned long long t = 0;
+    for (int w = 0; w < kBandWaves; ++w) t += part[w][h][k];
     if (dst && t) atomicAdd(dst, t);
   }
 }
@@ -1523,12 +1585,12 @@ int run_band(const StatsPlan &pl, int v, bool chain_done, const StatsWs &w, hipS
   }
   const int64_t items = small ? pl.nodes[v].cells / kChainChunk
                               : a.rows_out * (row_bits / kChainChunk);
-  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(ceil_div(items, 4), 4096)));
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(ceil_div(items, kBandWaves), 4096)));
   if (small)
-    hipLaunchKernelGGL(band_chain_small_kernel, grid, dim3(256), 0, stream,
+    hipLaunchKernelGGL(band_chain_small_kernel, grid, dim3(kBandThreads), 0, stream,
                        w.stack + pl.nodes[v].off / 4, a, w.stack + pl.nodes[run[H]].off / 4);
   else
-    hipLaunchKernelGGL(band_chain_kernel, grid, dim3(256), 0, stream,
+    hipLaunchKernelGGL(band_chain_kernel, grid, dim3(kBandThreads), 0, stream,
                        w.stack + pl.nodes[v].off / 4, a, w.stack + pl.nodes[run[H]].off / 4);
   EJ_LAUNCH_CHECK();
   *end = run[H];
@@ -1589,10 +1651,11 @@ int run_stats(const StatsPlan &pl, const StatsWs &w, const T *dense, int64_t n_d
     if (n.kind == kDenseRoot) {
       const bool vec = (reinterpret_cast<uintptr_t>(dense) % 16) == 0;
       const int64_t chunk = 4 * 64 * (16 / static_cast<int64_t>(sizeof(T)));
+      const int64_t blocks = ceil_div(ceil_div(n_dense, chunk), kBitsThreads / 64);
       hipLaunchKernelGGL(dense_bits_kernel<T>,
-                         dim3(static_cast<unsigned>(std::min<int64_t>(
-                             std::max<int64_t>(ceil_div(ceil_div(n_dense, chunk), 4), 1), 8192))),
-                         dim3(kBlock), 0, stream, dense, n_dense, vec, map,
+                         dim3(static_cast<unsigned>(
+                             std::min<int64_t>(std::max<int64_t>(blocks, 1), kBitsBlocks))),
+                         dim3(kBitsThreads), 0, stream, dense, n_dense, vec, map,
                          w.counts + r * kCountStride);
     } else {
       const int64_t words = static_cast<int64_t>(map_bytes(n.cells) / 4);
