@@ -335,9 +335,9 @@ def _measured_schemes(tensor, gpu_form) -> dict:
     with num_tuples and value_count counted on the GPU over the elements
     != 0 of gpu_form() for every tile shape in one call (the reference's
     _compute_sparsity_metrics, sparse.py:124-158 and dense.py:44-66)."""
-    schemes = {ts: TilingScheme(tensor, tensor.shape, ts) for ts in tensor.tile_shapes}
     form = gpu_form()
     if tensor.ndim == 0:
+        schemes = {ts: TilingScheme(tensor, tensor.shape, ts) for ts in tensor.tile_shapes}
         if form[0] == "coo":
             n = 1 if int(form[2].numel()) else 0
         else:
@@ -351,10 +351,7 @@ def _measured_schemes(tensor, gpu_form) -> dict:
         nt, vc = scheme_stats(tensor.tile_shapes, tensor.shape, indices=form[1], values=form[2])
     else:
         nt, vc = scheme_stats(tensor.tile_shapes, tensor.shape, dense=form[1])
-    for ts, n, v in zip(tensor.tile_shapes, nt, vc):
-        schemes[ts].num_tuples = n
-        schemes[ts].value_count = v
-    return schemes
+    return TilingScheme.measured(tensor, tensor.shape, tensor.tile_shapes, nt, vc)
 
 
 def _is_scipy(x) -> bool:

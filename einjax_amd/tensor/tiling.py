@@ -54,6 +54,23 @@ class TilingScheme:
         self.value_count = tuple(s // t for s, t in zip(self.shape, self.tile_shape))
         self.num_tuples = prod(self.value_count)
 
+    @classmethod
+    def measured(cls, node, shape: tuple, tile_shapes, num_tuples, value_counts) -> dict:
+        """tile_shape -> scheme with its statistics, for tile shapes and counts
+        that are tuples of ints already: a tensor has hundreds of schemes, and
+        filling the attributes at once takes a fifth of the constructor's
+        time (225 schemes of a 16384 x 16384 matrix: most of the host time of
+        its statistics)."""
+        out, new = {}, object.__new__
+        for ts, n, vc in zip(tile_shapes, num_tuples, value_counts):
+            out[ts] = s = new(cls)
+            s.__dict__ = {
+                "node": node, "shape": shape, "tile_shape": ts, "tile_size": prod(ts),
+                "value_count": vc, "num_tuples": n, "cost": 0.0, "comm": 0.0, "flops": 0.0,
+                "accumulated_cost": 0.0, "accumulated_comm": 0.0, "accumulated_flops": 0.0,
+                "source": (), "dependencies": set(), "partition_spec": None, "mesh_axes": None}
+        return out
+
     def __hash__(self):
         return hash((id(self.node), self.tile_shape))
 

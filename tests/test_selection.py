@@ -386,3 +386,15 @@ def test_relation_einsum_plan():
         plan("ii,ij->j", (2, 2), (2, 2))
     with pytest.raises(NotImplementedError):
         ej.einsum("ij,jk->ik", np.ones((2, 2)), np.ones((2, 2)))
+
+
+def test_measured_schemes_equal_constructed_ones():
+    shape = (12, 8)
+    tss = T.enumerate_tile_shapes(shape)
+    made = {ts: T.TilingScheme("node", shape, ts) for ts in tss}
+    got = T.TilingScheme.measured("node", shape, tss, [s.num_tuples for s in made.values()],
+                                  [s.value_count for s in made.values()])
+    assert list(got) == tss
+    for ts in tss:
+        assert vars(got[ts]) == vars(made[ts]) and hash(got[ts]) == hash(made[ts])
+    assert got[tss[0]].dependencies is not got[tss[1]].dependencies
