@@ -934,50 +934,82 @@ struct SegOpBf16 {
 // c ^ (r & 7) ^ ((r >> 3) & 1)); rhs chunk [32][BN] (chunk c of k-row r at
 // c ^ 4 ((r >> 2) & 3), so the four lane groups of a read hit four bank
 // quarters).
-template <int BM_, int BN_>
+// The backward's layouts mirror the two: an rhs [n][k] (BT, 'ik,jk->ij') is
+// staged and read as the lhs above, an lhs [k][m] (AT, 'ij,ik->jk') as the rhs.
+template <int BM_, int BN_, bool AT_ = false, bool BT_ = false>
 struct SegOpF32 {
   using elem = float;
   using a_elem = float;
   using b_elem = float;
-  static constexpr bool kBf16 = false, kSplit = false, kSplitB = false, AT = false, BT = false;
+  static constexpr bool kBf16 = false, kSplit = false, kSplitB = false, AT = AT_, BT = BT_;
   static constexpr int BM = BM_, BN = BN_, BK = 32;
-  static constexpr int A_ROWB = BK * 4, CHA = A_ROWB / 16, A_BYTES = BM * A_ROWB;
-  static constexpr int B_ROWB = BN * 4, CHB = B_ROWB / 16, B_BYTES = BK * B_ROWB;
-  static_assert(CHA == 8 && CHB >= 8, "row widths");
+  static constexpr int A_ROWB = AT ? BM * 4 : BK * 4, CHA = A_ROWB / 16, A_BYTES = BM * BK * 4;
+  static constexpr int B_ROWB = BT ? BK * 4 : BN * 4, CHB = B_ROWB / 16, B_BYTES = BK * BN * 4;
+  static_assert((AT ? CHA >= 8 : CHA == 8) && (BT ? CHB == 8 : CHB >= 8), "row widths");
 
-  __device__ static int swa(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-  __device__ static int swb(int krow) { return CHB >= 16 ? 4 * ((krow >> 2) & 3) : 4 * ((krow >> 2) & 1); }
-
+  // Swizzles of k-rows and k-major chunks (CH 16-byte chunks per row).
+  __device__ static int swk(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+  template <int CH>
+  __device__ static int swm(int krow) {
+    return CH >= 16 ? 4 * ((krow >> 2) & 3) : 4 * ((krow >> 2) & 1);
+  }
+  __device__ static uint32_t krows_src(int blk, int lane, int64_t stride) {
+    const int row = blk * 8 + lane / 8;
+    return static_cast<uint32_t>(row * stride + ((lane % 8) ^ swk(row)) * 4);
+  }
+  template <int CH>
+  __device__ static uint32_t kmajor_src(int blk, int lane, int64_t stride) {
+    const int krow = blk * (64 / CH) + lane / CH;
+    return static_cast<uint32_t>(krow * stride + ((lane % CH) ^ swm<CH>(krow)) * 4);
+  }
   __device__ static uint32_t a_src(int blk, int lane, const GemmGeom &g) {
-    const int row = blk * (1024 / A_ROWB) + lane / CHA;
-    const int c = (lane % CHA) ^ swa(row);
-    return static_cast<uint32_t>(row * g.a_sm + c * 4);
+    if constexpr (AT) return kmajor_src<CHA>(blk, lane, g.a_sk);
+    else return krows_src(blk, lane, g.a_sm);
   }
   __device__ static uint32_t b_src(int blk, int lane, const GemmGeom &g) {
-    const int krow = blk * (1024 / B_ROWB) + lane / CHB;
-    const int c = (lane % CHB) ^ swb(krow);
-    return static_cast<uint32_t>(krow * g.b_sk + c * 4);
+    if constexpr (BT) return krows_src(blk, lane, g.b_sn);
+    else return kmajor_src<CHB>(blk, lane, g.b_sk);
   }
 
-  // Per-lane LDS read offsets (rd[h], h = 0, 1: lhs chunk 4h + g of row
-  // row0 + (lane & 15); rd[2 + j]: column wcol + 16j + (lane & 15) of k-row
-  // 4g).  The MFMA loop is seg_gemm_kernel's.
+  // Per-lane LDS read offsets, lhs first.  A k-rows operand has two (h = 0, 1:
+  // chunk 4h + g of row row0 + (lane & 15); fragment f is 16 rows further), a
+  // k-major one has one per fragment (k-row 4g of its column; k-rows
+  // 16h + 4g + c share its swizzle).  The MFMA loop is seg_gemm_kernel's.
+  template <int FM>
+  static constexpr int n_ra = AT ? FM : 2;
+  template <int FN>
+  static constexpr int n_rb = BT ? 2 : FN;
   template <int FM, int FN>
-  static constexpr int n_rd = 2 + FN;
+  static constexpr int n_rd = n_ra<FM> + n_rb<FN>;
+
+  __device__ static uint32_t krows_rd(int row0, int h, int lane) {
+    const int row = row0 + (lane & 15);
+    return static_cast<uint32_t>(row * BK * 4 + ((4 * h + (lane >> 4)) ^ swk(row)) * 16);
+  }
+  template <int CH>
+  __device__ static uint32_t kmajor_rd(int col0, int lane) {
+    const int col = col0 + (lane & 15), krow = 4 * (lane >> 4);
+    return static_cast<uint32_t>(krow * CH * 16 + ((col >> 2) ^ swm<CH>(krow)) * 16 +
+                                 (col & 3) * 4);
+  }
 
   template <int FM, int FN>
   __device__ static void read_offsets(uint32_t (&rd)[n_rd<FM, FN>], int row0, int wcol,
                                       uint32_t b_region, int lane) {
-    const int row = row0 + (lane & 15), g = lane >> 4;
+    if constexpr (AT) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      rd[h] = static_cast<uint32_t>(row * A_ROWB + (((4 * h + g) ^ swa(row)) * 16));
+      for (int i = 0; i < FM; ++i) rd[i] = kmajor_rd<CHA>(row0 + i * 16, lane);
+    } else {
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int col = wcol + j * 16 + (lane & 15);
-      const int krow = 4 * g;  // rows 16h + 4g + c share this swizzle
-      rd[2 + j] = b_region + static_cast<uint32_t>(krow * B_ROWB +
-                                                   (((col >> 2) ^ swb(krow)) * 16) + (col & 3) * 4);
+      for (int h = 0; h < 2; ++h) rd[h] = krows_rd(row0, h, lane);
+    }
+    constexpr int o = n_ra<FM>;
+    if constexpr (BT) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) rd[o + h] = b_region + krows_rd(wcol, h, lane);
+    } else {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) rd[o + j] = b_region + kmajor_rd<CHB>(wcol + j * 16, lane);
     }
   }
 };
@@ -1546,20 +1578,42 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
                 acc[i][j], 0, 0, 0);
       } else {
         constexpr int A_ROWB = Op::A_ROWB, B_ROWB = Op::B_ROWB;
+        constexpr int RA = Op::template n_ra<FM>;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          f32x4_t af[FM];
-          float bv[FN][4];
+          float af[FM][4], bv[FN][4];
+          if constexpr (Op::AT) {
 #pragma unroll
-          for (int i = 0; i < FM; ++i)
-            af[i] = *reinterpret_cast<const f32x4_t *>((lds_ptr)(size_t)(base + rd[h]) +
-                                                      i * 16 * A_ROWB);
+            for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
+              for (int c = 0; c < 4; ++c)
+                af[i][c] = *reinterpret_cast<const float *>((lds_ptr)(size_t)(base + rd[i]) +
+                                                           (16 * h + c) * A_ROWB);
+          } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-              bv[j][c] = *reinterpret_cast<const float *>((lds_ptr)(size_t)(base + rd[2 + j]) +
-                                                         (16 * h + c) * B_ROWB);
+            for (int i = 0; i < FM; ++i) {
+              const f32x4_t x = *reinterpret_cast<const f32x4_t *>(
+                  (lds_ptr)(size_t)(base + rd[h]) + i * 16 * A_ROWB);
+#pragma unroll
+              for (int c = 0; c < 4; ++c) af[i][c] = x[c];
+            }
+          }
+          if constexpr (Op::BT) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+              const f32x4_t x = *reinterpret_cast<const f32x4_t *>(
+                  (lds_ptr)(size_t)(base + rd[RA + h]) + j * 16 * B_ROWB);
+#pragma unroll
+              for (int c = 0; c < 4; ++c) bv[j][c] = x[c];
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+              for (int c = 0; c < 4; ++c)
+                bv[j][c] = *reinterpret_cast<const float *>((lds_ptr)(size_t)(base + rd[RA + j]) +
+                                                           (16 * h + c) * B_ROWB);
+          }
 #pragma unroll
           for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -1848,7 +1902,15 @@ int launch_gemm_layout(bool a_direct, bool b_direct, const void *A, const void *
   const T *a = static_cast<const T *>(A);
   const T *b = static_cast<const T *>(B);
   dim3 grid(static_cast<unsigned>(nblk)), block(256);
-  if (a_direct && b_direct)
+  if constexpr (sizeof(T) == 4 && BK == 32) {  // the ring kernels take the other layouts
+    if (a_direct || !b_direct) {
+      set_error("no register-staged fp32 GEMM for this layout");
+      return EJ_E_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL((tile_gemm_kernel<T, BM, BN, BK, false, true>), grid, block, 0, stream, a, b, C, src, g);
+    EJ_LAUNCH_CHECK();
+    return EJ_OK;
+  } else if (a_direct && b_direct)
     hipLaunchKernelGGL((tile_gemm_kernel<T, BM, BN, BK, true, true>), grid, block, 0, stream, a, b, C, src, g);
   else if (a_direct)
     hipLaunchKernelGGL((tile_gemm_kernel<T, BM, BN, BK, true, false>), grid, block, 0, stream, a, b, C, src, g);
@@ -1996,6 +2058,22 @@ int launch_seg_gemm_f32(int bm, int bn, int grp, const void *A, const void *B, v
   return EJ_E_UNSUPPORTED;
 }
 
+// The same with an [n][k] rhs (AT = false, BT = true) or a [k][m] lhs (AT =
+// true, BT = false), one segment per workgroup.
+template <bool AT, bool BT>
+int launch_seg_gemm_f32_t(int bm, int bn, const void *A, const void *B, void *C,
+                          const PairSrc &src, const GemmGeom &g, int64_t n_seg,
+                          hipStream_t stream) {
+#define EJ_F32_CASE(M_, N_, WGM_)  \
+  if (bm == M_ && bn == N_)        \
+    return launch_seg_gemm_t<SegOpF32<M_, N_, AT, BT>, 1, WGM_, 4>(A, B, C, src, g, n_seg, stream);
+  EJ_F32_CASE(32, 32, 2) EJ_F32_CASE(32, 64, 2) EJ_F32_CASE(64, 32, 2)
+  EJ_F32_CASE(64, 64, 2) EJ_F32_CASE(128, 32, 4) EJ_F32_CASE(128, 64, 2)
+#undef EJ_F32_CASE
+  set_error("no fp32 segment GEMM configuration for %dx%d", bm, bn);
+  return EJ_E_UNSUPPORTED;
+}
+
 int pick_block(int64_t x) { return x % 128 == 0 ? 128 : x % 64 == 0 ? 64 : x % 32 == 0 ? 32 : 0; }
 
 // Segments per workgroup of the fused kernel that try_gemm picks for a
@@ -2105,16 +2183,19 @@ bool try_gemm(const ej_einsum_desc *d, int32_t dtype, const void *A, const void 
     }
     return true;
   }
-  // fp32, k-contiguous lhs, n-contiguous rhs, K a multiple of 32, 16-byte
-  // rows: the LDS-ring kernel with fp32 MFMAs (grouped like the bf16 one).
-  if (dtype == EJ_F32 && ad && !bd && d->k % 32 == 0 && d->b_sn == 1 && d->b_sk % 4 == 0 &&
+  // fp32, K a multiple of 32, 16-byte rows, at least one operand in the layout
+  // the forward has: the LDS-ring kernel with fp32 MFMAs (the forward's layout
+  // grouped like the bf16 one).
+  if (dtype == EJ_F32 && (ad || !bd) && d->k % 32 == 0 &&
       (bm == 32 || bm == 64 || bm == 128) && src.n_a_tiles < (int64_t(1) << 31) &&
       src.n_b_tiles < (int64_t(1) << 31)) {
     const int fbn = d->n % 64 == 0 ? 64 : 32;
     if (d->n % fbn == 0) {
       g.nblocks = d->n / fbn;
       const bool grouped = src.seg_off && d->seg_group > 0 && d->seg_group % 4 == 0;
-      *status = launch_seg_gemm_f32(bm, fbn, grouped ? 4 : 1, A, B, C, src, g, n_seg, stream);
+      *status = !ad  ? launch_seg_gemm_f32_t<true, false>(bm, fbn, A, B, C, src, g, n_seg, stream)
+                : bd ? launch_seg_gemm_f32_t<false, true>(bm, fbn, A, B, C, src, g, n_seg, stream)
+                     : launch_seg_gemm_f32(bm, fbn, grouped ? 4 : 1, A, B, C, src, g, n_seg, stream);
       return true;
     }
   }

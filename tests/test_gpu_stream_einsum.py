@@ -150,3 +150,26 @@ def test_pair_results_in_lines(gpu, m, k, n, spec):
         _device.ptr(dli), _device.ptr(dri), len(li), _device.ptr(flat[1:]),
         _device.stream_ptr()) == _lib.EJ_OK
     assert torch.equal(flat[1:].view(got.shape), got)
+
+
+@pytest.mark.parametrize("spec", ["ij,kj->ik", "ji,jk->ik"])
+@pytest.mark.parametrize("m,k,n", [(32, 32, 32), (64, 64, 64), (128, 32, 128), (96, 160, 32),
+                                   (32, 64, 192), (192, 96, 96)])
+def test_fp32_ring_transposed_layouts(gpu, spec, m, k, n):
+    """The backward's fp32 layouts on blocked extents: every block shape, one
+    and several K stages, segments of zero to many pairs (one and several to a
+    workgroup), an invalid pair, NaN tiles that no pair names."""
+    print("[case] fp32 ring", spec, m, k, n, flush=True)
+    for pairs, segs in ((40, 9), (150, 2100)):
+        lt, rt, lv, rv, li, ri, perm, off = _case(spec, m, k, n, torch.float32, m + k + n,
+                                                  pairs=pairs, segs=segs)
+        li[li == 3], ri[ri == 5] = 2, 4
+        pv = R.kernel_einsum(lv, rv, li, ri, spec, precision="fp64")
+        lv[3], rv[5] = np.nan, np.nan
+        li[7] = len(lv)
+        pv[7] = 0
+        pv = pv[perm]
+        want = np.stack([pv[a:b].sum(0) for a, b in zip(off[:-1], off[1:])])
+        got = _run(spec, lt, rt, lv, rv, li, ri, perm, off, torch.float32)
+        longest = int(np.diff(off).max()) * k
+        assert R.rel_l2(got.cpu().numpy(), want) <= _tol(torch.float32, torch.float32, longest)
