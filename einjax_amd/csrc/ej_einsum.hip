@@ -1406,9 +1406,13 @@ __global__ __launch_bounds__(NW * 64, 2) void seg_gemm_kernel(const typename Op:
           for (int r = 0; r < LR; ++r)
             put_out(reinterpret_cast<uint16_t *>(st + ((lane >> 4) * LR + r) * LROW) + j * 16 +
                         (lane & 15), acc[i][j][r0 + r]);
+        // A wave's LDS accesses run in program order; the strip is written and
+        // read under different types, so the compiler is held to that order.
+        asm volatile("" ::: "memory");
         const int x = lane / LPR, ch = lane % LPR;
         const uint2 lo = *reinterpret_cast<const uint2 *>(st + x * LROW + ch * 16);
         const uint2 hi = *reinterpret_cast<const uint2 *>(st + x * LROW + ch * 16 + 8);
+        asm volatile("" ::: "memory");
         const int row = i * 16 + x / LR * 4 + r0 + x % LR;
         *reinterpret_cast<uint4 *>(cb + row * csm + ch * 8) = make_uint4(lo.x, lo.y, hi.x, hi.y);
       }
