@@ -25,9 +25,12 @@
 // W waves share a segment: wave w takes K blocks w, w + W, ... of the
 // segment's whole run of pairs, so the waves are balanced for every number of
 // fragments and of pairs, need no barrier while they stream, and add their
-// blocks once at the end through LDS, in wave order (results are
-// deterministic).  W = 4 where there are too few output blocks to fill the
-// chip, W = 1 (four segments to a workgroup, no LDS) otherwise.
+// blocks once at the end through LDS, in wave order.  W = 4 where there are
+// too few output blocks to fill the chip, W = 1 (four output blocks to a
+// workgroup, LDS unused) otherwise.  The two add a segment's K blocks in
+// different orders, so the choice is made on the device from the segments
+// that are there, never from the bound a launch is sized for: an einsum then
+// gives the same bits whether its plan was counted first or queued.
 // Measured (one MI355X), against one thread per output element: block-sparse
 // 6000^2 x dense 6000 x 1500 fp32, 75 x 75 tiles (12,800 pairs, 10.8 GFLOP)
 // 170 us / 3,380 us: 64 TFLOP/s, bound by the fp32 MFMAs (48% busy; the last
@@ -35,6 +38,8 @@
 // bf16, 80 x 80 tiles (5,240 pairs) 32 us / 1,750 us, bound by the latency of
 // one or two K blocks per wave.
 #pragma once
+
+#include <algorithm>
 
 #include "ej_gemm.h"
 
@@ -262,10 +267,20 @@ __device__ inline void stream_put(uint16_t *p, const float *v) {
 // packed fragments.  Large blocks get two waves per SIMD, small ones more.
 constexpr int stream_waves(int nf) { return nf >= 15 ? 2 : nf >= 9 || nf == 5 ? 3 : 4; }
 
+// Below this many output blocks four waves share each.  2048 is the chip's
+// wave slots at two waves per SIMD: fewer blocks cannot fill it one wave each.
+// Measured, one wave / four waves a block: 80 x 80 bf16, ~4,500 blocks of 1.2
+// pairs 32 / 73 us (most of a split block's time is its reduction); 120 x 120
+// bf16, 4,592 blocks 25 / 31 us; 75 x 75 fp32, 1,600 blocks of 8 pairs 219 /
+// 170 us; 36 x 36 fp32, 252 blocks of up to 50 pairs 58 / 19 us.
+constexpr int64_t kStreamSplitBlocks = 2048;
+
+// Output block lb (uniform over the wave) of the launch; `part`: the W = 4
+// reduction's LDS.  Every wave of a W = 4 workgroup calls it with one lb.
 template <typename T, int FM, int FN, int AMODE, int BMODE, int W>
-__global__ __launch_bounds__(256, stream_waves(FM * FN)) void stream_gemm_kernel(
-    const T *__restrict__ A, const T *__restrict__ B, void *__restrict__ C, PairSrc src, GemmGeom g,
-    int64_t n_seg) {
+__device__ inline void stream_block(const T *__restrict__ A, const T *__restrict__ B,
+                                    void *__restrict__ C, const PairSrc &src, const GemmGeom &g,
+                                    uint32_t lb, float *part) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using OA = StreamOp<T, FM, AMODE>;
   using OB = StreamOp<T, FN, BMODE>;
@@ -274,20 +289,6 @@ __global__ __launch_bounds__(256, stream_waves(FM * FN)) void stream_gemm_kernel
   constexpr int NF = FM * FN;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-  // Output block of this workgroup (W = 4) or wave (W = 1).
-  const int64_t per_seg = g.nblocks * g.mblocks * g.batch;
-  int64_t nseg = n_seg;
-  if (src.n_live) {
-    const int64_t nl = ld_uniform(src.n_live, 0);
-    nseg = nl < nseg ? nl : nseg;
-  }
-  constexpr int UPB = 4 / W;  // output blocks per workgroup
-  const uint32_t units = static_cast<uint32_t>(nseg * per_seg);  // below 2^31 (launch_stream_t)
-  const uint32_t live = (units + UPB - 1) / UPB;
-  if (blockIdx.x >= live) return;
-  const uint32_t lb = xcd_logical_block(live, kXcdRun) * UPB + (W == 1 ? wave : 0);
-  if (lb >= units) return;  // W = 1 only: no barrier follows
   const BlockPos at_block = block_pos(lb, g);
   const int nb = static_cast<int>(at_block.nb), mb = static_cast<int>(at_block.mb);
   const int64_t bi = at_block.bi, seg = at_block.seg;
@@ -447,7 +448,6 @@ __global__ __launch_bounds__(256, stream_waves(FM * FN)) void stream_gemm_kernel
     // Wave r sums and stores result rows 4 gq + r of every fragment: each wave
     // hands the other three their rows through LDS (one float per lane and
     // fragment, consecutive lanes on consecutive banks).
-    __shared__ float part[4 * 3 * NF * 64];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if (r == wave) continue;
@@ -486,6 +486,34 @@ __global__ __launch_bounds__(256, stream_waves(FM * FN)) void stream_gemm_kernel
 #endif
 }
 
+template <typename T, int FM, int FN, int AMODE, int BMODE>
+__global__ __launch_bounds__(256, stream_waves(FM * FN)) void stream_gemm_kernel(
+    const T *__restrict__ A, const T *__restrict__ B, void *__restrict__ C, PairSrc src, GemmGeom g,
+    int64_t n_seg) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ float part[4 * 3 * FM * FN * 64];
+  int64_t nseg = n_seg;
+  if (src.n_live) {
+    const int64_t nl = ld_uniform(src.n_live, 0);
+    nseg = nl < nseg ? nl : nseg;
+  }
+  // below 2^31 (try_stream)
+  const uint32_t units = static_cast<uint32_t>(nseg * (g.nblocks * g.mblocks * g.batch));
+  if (units < kStreamSplitBlocks) {
+    if (blockIdx.x >= units) return;
+    stream_block<T, FM, FN, AMODE, BMODE, 4>(A, B, C, src, g, xcd_logical_block(units, kXcdRun),
+                                             part);
+  } else {
+    const uint32_t live = (units + 3) / 4;
+    if (blockIdx.x >= live) return;
+    const uint32_t lb = xcd_logical_block(live, kXcdRun) * 4 +
+                        __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (lb >= units) return;
+    stream_block<T, FM, FN, AMODE, BMODE, 1>(A, B, C, src, g, lb, part);
+  }
+#endif
+}
+
 // Fragments per wave along an extent: the extent's fragments split evenly
 // over the fewest blocks of at most five.
 inline int stream_frags(int64_t ext) {
@@ -499,34 +527,23 @@ int launch_stream_f32(int amode, int bmode, const void *A, const void *B, void *
 int launch_stream_bf16(int amode, int bmode, const void *A, const void *B, void *C,
                        const PairSrc &src, GemmGeom g, int64_t n_seg, hipStream_t stream);
 
-// Below this many output blocks four waves share each.  2048 is the chip's
-// wave slots at two waves per SIMD: fewer blocks cannot fill it one wave each.
-// Measured, one wave / four waves a block: 80 x 80 bf16, ~4,500 blocks of 1.2
-// pairs 32 / 73 us (most of a split block's time is its reduction); 120 x 120
-// bf16, 4,592 blocks 25 / 31 us; 75 x 75 fp32, 1,600 blocks of 8 pairs 219 /
-// 170 us; 36 x 36 fp32, 252 blocks of up to 50 pairs 58 / 19 us.
-constexpr int64_t kStreamSplitBlocks = 2048;
-
 template <typename T, int FM, int FN, int AMODE, int BMODE>
 int launch_stream_t(const void *A, const void *B, void *C, const PairSrc &src, GemmGeom g,
                     int64_t n_seg, hipStream_t stream) {
   g.mblocks = ceil_div(g.m, FM * 16);
   g.nblocks = ceil_div(g.n, FN * 16);
+  // One workgroup per output block below the split, one per four from it on; a
+  // bound's live blocks may fall on either side.
   const int64_t units = n_seg * g.mblocks * g.nblocks * g.batch;
-  const bool split = units < kStreamSplitBlocks;
-  const int64_t nblk = split ? units : ceil_div(units, 4);
-  if (nblk >= (int64_t(1) << 31)) {
+  int64_t nblk = units < kStreamSplitBlocks ? units : ceil_div(units, 4);
+  if (src.n_live && units >= kStreamSplitBlocks) nblk = std::max(nblk, kStreamSplitBlocks - 1);
+  if (units >= (int64_t(1) << 31)) {
     set_error("einsum launch too large");
     return EJ_E_UNSUPPORTED;
   }
-  const dim3 grid(static_cast<unsigned>(nblk));
-  const T *a = static_cast<const T *>(A), *b = static_cast<const T *>(B);
-  if (split)
-    hipLaunchKernelGGL((stream_gemm_kernel<T, FM, FN, AMODE, BMODE, 4>), grid, dim3(256), 0,
-                       stream, a, b, C, src, g, n_seg);
-  else
-    hipLaunchKernelGGL((stream_gemm_kernel<T, FM, FN, AMODE, BMODE, 1>), grid, dim3(256), 0,
-                       stream, a, b, C, src, g, n_seg);
+  hipLaunchKernelGGL((stream_gemm_kernel<T, FM, FN, AMODE, BMODE>),
+                     dim3(static_cast<unsigned>(nblk)), dim3(256), 0, stream,
+                     static_cast<const T *>(A), static_cast<const T *>(B), C, src, g, n_seg);
   EJ_LAUNCH_CHECK();
   return EJ_OK;
 }

@@ -1,6 +1,8 @@
 """Tile einsums on extents the blocked MFMA kernels do not take (the streaming
 GEMM): every number of 16-wide fragments and its edges, K tails, all operand
-layouts, one and four waves per output block, against float64."""
+layouts, one and four waves per output block, against float64; the same bits on every path that plans an einsum."""
+
+import ctypes
 
 import numpy as np
 import pytest
@@ -8,7 +10,9 @@ import torch
 
 from oracle import reference_path as R
 
-from einjax_amd import _device
+import einjax_amd as ej
+from einjax_amd import _device, _lib
+from einjax_amd.execution.engine import ContractionPlan, ContractionStep
 
 pytestmark = pytest.mark.gpu
 
@@ -84,6 +88,97 @@ def test_many_pairs_one_wave_each(gpu, m, k, n, spec, dtype):
         assert R.rel_l2(got.float().cpu().numpy(), ref) <= _tol(dtype, dtype, k)
 
 
+def _segment_sums(lv, rv, li, ri, perm, off, spec):
+    """float64 segment sums on the GPU; a pair with an index out of range adds nothing."""
+    ok = (li >= 0) & (li < len(lv)) & (ri >= 0) & (ri < len(rv))
+    pv = R.kernel_einsum(lv, rv, np.where(ok, li, 0), np.where(ok, ri, 0), spec, precision="fp64")
+    pv[~ok] = 0
+    pv = pv[perm]
+    return np.stack([pv[a:b].sum(0) for a, b in zip(off[:-1], off[1:])])
+
+
+@pytest.mark.parametrize("live", [0, 1, 200, 2047, 2048, 2600])
+@pytest.mark.parametrize("t,dtype", [(40, torch.float32), (20, torch.bfloat16)])
+def test_segment_bound(gpu, t, dtype, live):
+    """A launch sized for 2,600 segments of 0 to several pairs of which `live`
+    are there: bitwise the launch of exactly those, float64 within rounding,
+    nothing written past them."""
+    print("[case] stream bound", t, dtype, live, flush=True)
+    rng = np.random.default_rng(live)
+    bound, pairs = 2600, 6000
+    lt, rt, lv, rv, li, ri, perm, _ = _case("ij,jk->ik", t, t, t, dtype, 9, pairs=pairs)
+    off = np.sort(rng.integers(0, pairs, bound + 1)).astype(np.int32)
+    off[3] = off[2]
+    li[5], ri[11] = len(lv), -1
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    a, b, dli, dri, dperm, doff = (dev(lv).to(dtype), dev(rv).to(dtype), dev(li), dev(ri),
+                                   dev(perm), dev(off))
+    desc = _device.describe("ij,jk->ik", lt, rt)
+    out = torch.full((bound, t, t), 7.0, device="cuda")
+    desc.out_dtype = _lib.EJ_F32
+    nlive = torch.tensor([live], dtype=torch.int64, device="cuda")
+    assert _lib.load().ej_segment_einsum_async(
+        ctypes.byref(desc), _lib.EJ_BF16 if dtype == torch.bfloat16 else _lib.EJ_F32,
+        _device.ptr(a), _device.ptr(b), a.shape[0], b.shape[0], _device.ptr(dli),
+        _device.ptr(dri), _device.ptr(dperm), _device.ptr(doff), bound, _device.ptr(nlive), None,
+        0, _device.ptr(out), _device.stream_ptr()) == _lib.EJ_OK
+    assert bool((out[live:] == 7.0).all())
+    if live == 0:
+        return
+    exact = _device.segment_einsum(desc, a, b, dli, dri, dperm, doff[:live + 1].contiguous(),
+                                   torch.float32)
+    assert torch.equal(out[:live], exact)
+    want = _segment_sums(lv, rv, li, ri, perm, off[:live + 1], "ij,jk->ik")
+    longest = max(int(np.diff(off[:live + 1]).max()), 1) * t
+    assert R.rel_l2(exact.cpu().numpy(), want) <= _tol(dtype, torch.float32, longest)
+
+
+def _relation(rng, keep, t, dtype):
+    c = np.ascontiguousarray(np.argwhere(keep), dtype=np.int32)
+    v = torch.from_numpy(rng.standard_normal((len(c), t, t)).astype(np.float32)).cuda().to(dtype)
+    return ej.SparseTensorRelation(torch.from_numpy(c).cuda(), v,
+                                   tuple(g * t for g in keep.shape), (t, t))
+
+
+@pytest.mark.parametrize("rhs", ["sparse", "dense"])
+@pytest.mark.parametrize("t,dtype", [(40, torch.float32), (75, torch.float32), (80, torch.bfloat16)])
+def test_same_bits_on_every_path(gpu, t, dtype, rhs):
+    """Fewer output tiles than the split's 2,048, bounds above it: the plan
+    counted first, the row or dense plan, the prepared step, the queued plan,
+    an engine step on new relations, all bitwise alike (fp32 results)."""
+    print("[case] stream paths", t, dtype, rhs, flush=True)
+    rng = np.random.default_rng(t)
+    if rhs == "sparse":  # about 2,800 pairs, 1,700 output tiles, bound 2,500
+        ka, kb = rng.random((50, 50)) < 0.15, rng.random((50, 50)) < 0.15
+        ka[7], kb[9] = False, False
+    else:  # 60 lhs tiles in 40 of 70 rows, 40 rhs columns: 1,600 output tiles, bound 2,400
+        ka, kb = np.zeros((70, 12), bool), np.ones((12, 40), bool)
+        rows = rng.permutation(70)[:40]
+        ka[rows, rng.integers(0, 6, 40)] = True
+        ka[rows[:20], rng.integers(6, 12, 20)] = True
+    L, Rr = _relation(rng, ka, t, dtype), _relation(rng, kb, t, dtype)
+    join, spec, agg = [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)]
+    li, ri = ej.coordinate_join(L, Rr, join)
+    coords, offsets, perm, _ = _device.segment_plan(L.coords, Rr.coords, li, ri, agg,
+                                                    [ka.shape[0], kb.shape[1]])
+    P, U = li.numel(), coords.shape[0]
+    assert P > 2048 > U and int(torch.diff(offsets).max()) > 1
+    desc = _device.describe(spec, (t, t), (t, t))
+    want = _device.segment_einsum(desc, L.values, Rr.values, li, ri, perm, offsets, torch.float32)
+    for call in range(3):  # counted first (or the dense plan), then queued, then prepared
+        got = ej.execute_sparse(L, Rr, join, spec, agg, out_dtype=torch.float32)
+        assert torch.equal(got.coords, coords) and torch.equal(got.values, want), call
+    status, res = _device.queued_segment_einsum(
+        L.coords, Rr.coords, join, [kb.shape[0]], agg, [ka.shape[0], kb.shape[1]],
+        _device.describe(spec, (t, t), (t, t)), L.values, Rr.values, 4 * P, torch.float32)
+    assert status == "ok" and torch.equal(res[4], want)
+    anew = [ej.SparseTensorRelation(r.coords.clone(), r.values.clone(), r.shape, r.tile_shape)
+            for r in (L, Rr)]
+    engine = ej.ExecutionEngine(out_dtype=torch.float32)
+    got = engine.execute_plan(ContractionPlan(spec, [ContractionStep(0, spec, (0, 1))]), anew)
+    assert torch.equal(got.coords, coords) and torch.equal(got.values, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("spec", ["ij,jk->ik", "ij,kj->ik", "ji,jk->ik", "ji,kj->ik"])
 def test_neighbour_tiles_and_invalid_pairs(gpu, spec, dtype):
@@ -130,9 +225,6 @@ def test_pair_results_in_lines(gpu, m, k, n, spec):
     results), as they come (fp32 results, transposed results, an output that is
     not 16-byte aligned): all of them one fp32 result, rounded once."""
     print("[case] pair lines", spec, m, k, n, flush=True)
-    from einjax_amd import _lib
-    import ctypes
-
     lt, rt, lv, rv, li, ri, _, _ = _case("ij,jk->ik", m, k, n, torch.bfloat16, m + k + n)
     li[3] = len(lv)  # out of range: a tile of zeros
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
