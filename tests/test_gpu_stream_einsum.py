@@ -1,6 +1,7 @@
 """Tile einsums on extents the blocked MFMA kernels do not take (the streaming
 GEMM): every number of 16-wide fragments and its edges, K tails, all operand
-layouts, one and four waves per output block, against float64; the same bits on every path that plans an einsum."""
+layouts, one and four waves per output block, short and long segments, against
+float64; the same bits on every path that plans an einsum."""
 
 import ctypes
 
@@ -75,7 +76,7 @@ def test_segments(gpu, spec, m, k, n, dtype):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_many_pairs_one_wave_each(gpu, m, k, n, spec, dtype):
     """Per-pair results of more pairs than split blocks, and of a few of them
-    (four waves): within rounding of float64, and the two splits of each other."""
+    (four waves), both within rounding of float64."""
     print("[case] stream pairs", spec, m, k, n, dtype, flush=True)
     lt, rt, lv, rv, li, ri, _, _ = _case(spec, m, k, n, dtype, 3, pairs=2500)
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
@@ -95,6 +96,25 @@ def _segment_sums(lv, rv, li, ri, perm, off, spec):
     pv[~ok] = 0
     pv = pv[perm]
     return np.stack([pv[a:b].sum(0) for a, b in zip(off[:-1], off[1:])])
+
+
+@pytest.mark.parametrize("spec,m,k,n", [("ij,jk->ik", 20, 37, 33), ("ij,kj->ik", 75, 21, 18),
+                                        ("ji,jk->ik", 33, 40, 50)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_long_segments(gpu, spec, m, k, n, dtype):
+    """Segments of more pairs than a wave's lanes hold (64 at a time): 63 to
+    129 and 300 pairs, invalid pairs on both sides of a reload."""
+    print("[case] stream long segments", spec, m, k, n, dtype, flush=True)
+    lens = [63, 64, 65, 0, 128, 129, 1, 300]
+    off = np.cumsum([0] + lens).astype(np.int32)
+    lt, rt, lv, rv, li, ri, perm, _ = _case(spec, m, k, n, dtype, 5, pairs=int(off[-1]))
+    li[perm[off[2] + 63]], ri[perm[off[2] + 64]], li[perm[off[7] + 191]] = -1, len(rv), len(lv)
+    want = _segment_sums(lv, rv, li, ri, perm, off, spec)
+    got = _run(spec, lt, rt, lv, rv, li, ri, perm, off, dtype, torch.float32).cpu().numpy()
+    assert R.rel_l2(got, want) <= _tol(dtype, torch.float32, 300 * k)
+    for u, x in enumerate(lens):
+        assert R.rel_l2(got[u], want[u]) <= _tol(dtype, torch.float32, max(x, 1) * k), u
+    assert not got[3].any()
 
 
 @pytest.mark.parametrize("live", [0, 1, 200, 2047, 2048, 2600])
