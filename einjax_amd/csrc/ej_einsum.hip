@@ -1794,55 +1794,55 @@ __global__ __launch_bounds__(256) void generic_einsum_kernel(const T *__restrict
 // output, in the same order), summed over the segment's pairs.
 //
 // Bound by memory: both tiles read once, the result written once.  A thread
-// takes up to four 16-byte vectors of each operand, all loaded before the
-// first product, so a workgroup has 32 KB in flight; consecutive threads on
-// consecutive vectors.  Tiles whose size is no multiple of 16 bytes put later
-// tiles off alignment: the vectors are then read and written unaligned, the
-// last partial one element by element.  The generic kernel, one element and a
-// division per output label a thread, took 33 us on 1,434 pairs of 64 x 64
-// fp32 tiles (71 MB), this one 12.5 us (5.6 TB/s).
-constexpr int kEwiseVecs = 4;  // 16-byte vectors per thread
-
+// takes V 16-byte vectors of each operand, all loaded before the first
+// product, so a workgroup has 32 KB in flight at V = 4; consecutive threads on
+// consecutive vectors.  A tile's last vector ends with the tile: where the tile
+// is no whole number of vectors it overlaps its neighbour, whose elements are
+// then formed and written twice, alike.  Such tiles also put later ones off
+// alignment: vectors are read and written at the elements' alignment.
+// 1,434 pairs of 64 x 64 fp32 tiles (71 MB): 12.5 us (5.6 TB/s); the generic
+// kernel, one element and a division per output label a thread, 33 us.
+// A tile's vectors are split evenly over the fewest workgroups of at most four
+// a thread (small tiles: one workgroup of one a thread, bound by the latency of
+// the segment's indices and loads).  20,000 pairs in 12,000 segments, fp32 and
+// bf16, the generic kernel's time in brackets: 16 elements 11 and 12 us (14,
+// 13), 256 elements 12 and 11 us (23, 23), 4,096 elements 86 and 33 us (252,
+// 254).
 template <typename T>
-struct EwiseVec {
-  static constexpr int N = 16 / sizeof(T);
-  T v[N];
-};
+constexpr int kEwiseN = 16 / static_cast<int>(sizeof(T));  // elements per vector
 
-template <typename T, class Ar>
+template <typename T, class Ar, int V>
 __global__ __launch_bounds__(256) void ewise_kernel(const T *__restrict__ A,
                                                     const T *__restrict__ B, void *__restrict__ C,
                                                     PairSrc src, int64_t elems, int64_t eblocks,
                                                     int32_t out_bf16) {
   using Acc = typename Ar::acc;
-  constexpr int N = EwiseVec<T>::N;
+  constexpr int N = kEwiseN<T>;
   const int64_t seg = blockIdx.x / eblocks;
   if (seg_dead(src, seg)) return;
-  const int64_t e0 = ((blockIdx.x % eblocks) * kEwiseVecs * 256 + threadIdx.x) * N;
+  const int64_t e0 = ((blockIdx.x % eblocks) * V * 256 + threadIdx.x) * N;
+  if (e0 >= elems) return;
+  const int64_t last = elems - N;  // elems >= N (is_ewise)
   int64_t q0, q1;
   seg_range(src, seg, &q0, &q1);
-  Acc acc[kEwiseVecs][N] = {};
+  Acc acc[V][N] = {};
   for (int64_t q = q0; q < q1; ++q) {
     int64_t at, bt;
     if (!pair_tiles(src, q, &at, &bt)) continue;
     const T *a = A + at * elems, *b = B + bt * elems;
-    EwiseVec<T> x[kEwiseVecs], y[kEwiseVecs];
+    struct Vec {
+      T v[N];
+    } x[V], y[V];
 #pragma unroll
-    for (int u = 0; u < kEwiseVecs; ++u) {
+    for (int u = 0; u < V; ++u) {
+      // (past the tile: its last vector again, so that no branch parts the loads)
       const int64_t e = e0 + u * 256 * N;
-      if (e + N <= elems) {
-        __builtin_memcpy(&x[u], a + e, 16);
-        __builtin_memcpy(&y[u], b + e, 16);
-      } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          x[u].v[i] = e + i < elems ? a[e + i] : T(0);
-          y[u].v[i] = e + i < elems ? b[e + i] : T(0);
-        }
-      }
+      __builtin_memcpy(&x[u], a + (e < last ? e : last), 16);
+      __builtin_memcpy(&y[u], b + (e < last ? e : last), 16);
     }
+    __builtin_amdgcn_sched_barrier(0);  // all loads before the first product
 #pragma unroll
-    for (int u = 0; u < kEwiseVecs; ++u)
+    for (int u = 0; u < V; ++u)
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const Acc p = Ar::load(&x[u].v[i]) * Ar::load(&y[u].v[i]);
@@ -1851,44 +1851,55 @@ __global__ __launch_bounds__(256) void ewise_kernel(const T *__restrict__ A,
   }
   const int64_t c0 = seg * elems;
 #pragma unroll
-  for (int u = 0; u < kEwiseVecs; ++u) {
+  for (int u = 0; u < V; ++u) {
     const int64_t e = e0 + u * 256 * N;
-    if (e + N <= elems) {
-      // 16 bytes at a time (fp32 results of bf16 tiles: twice)
-      if (sizeof(T) == 2 && out_bf16) {
-        uint16_t h[N];
+    if (e >= elems) continue;
+    const int64_t c = c0 + (e < last ? e : last);
+    // 16 bytes at a time (fp32 results of bf16 tiles: twice)
+    if (sizeof(T) == 2 && out_bf16) {
+      uint16_t h[N];
 #pragma unroll
-        for (int i = 0; i < N; ++i) put_out(&h[i], static_cast<float>(acc[u][i]));
-        __builtin_memcpy(static_cast<uint16_t *>(C) + c0 + e, h, sizeof(h));
-      } else {
-        __builtin_memcpy(static_cast<Acc *>(C) + c0 + e, acc[u], sizeof(acc[u]));
-      }
+      for (int i = 0; i < N; ++i) put_out(&h[i], static_cast<float>(acc[u][i]));
+      __builtin_memcpy(static_cast<uint16_t *>(C) + c, h, sizeof(h));
     } else {
-#pragma unroll
-      for (int i = 0; i < N; ++i)
-        if (e + i < elems) Ar::store(C, c0 + e + i, acc[u][i], out_bf16 != 0);
+      __builtin_memcpy(static_cast<Acc *>(C) + c, acc[u], sizeof(acc[u]));
     }
   }
 }
 
-template <typename T, class Ar>
-int launch_ewise(const ej_einsum_desc *d, const void *A, const void *B, void *C,
-                 const PairSrc &src, int64_t n_seg, hipStream_t stream) {
-  const int64_t eb = ceil_div(d->c_elems, int64_t(256) * kEwiseVecs * EwiseVec<T>::N);
+template <typename T, class Ar, int V>
+int launch_ewise_v(const ej_einsum_desc *d, const void *A, const void *B, void *C,
+                   const PairSrc &src, int64_t n_seg, hipStream_t stream) {
+  const int64_t eb = ceil_div(d->c_elems, int64_t(256) * V * kEwiseN<T>);
   if (n_seg * eb >= (int64_t(1) << 31)) {
     set_error("einsum launch too large");
     return EJ_E_UNSUPPORTED;
   }
-  hipLaunchKernelGGL((ewise_kernel<T, Ar>), dim3(static_cast<unsigned>(n_seg * eb)), dim3(256), 0,
-                     stream, static_cast<const T *>(A), static_cast<const T *>(B), C, src,
+  hipLaunchKernelGGL((ewise_kernel<T, Ar, V>), dim3(static_cast<unsigned>(n_seg * eb)),
+                     dim3(256), 0, stream, static_cast<const T *>(A), static_cast<const T *>(B), C, src,
                      d->c_elems, eb, d->out_dtype == EJ_BF16 ? 1 : 0);
   EJ_LAUNCH_CHECK();
   return EJ_OK;
 }
 
-// Whether the einsum is an elementwise product of tiles of the same layout.
-bool is_ewise(const ej_einsum_desc *d) {
+template <typename T, class Ar>
+int launch_ewise(const ej_einsum_desc *d, const void *A, const void *B, void *C,
+                 const PairSrc &src, int64_t n_seg, hipStream_t stream) {
+  const int64_t nvec = ceil_div(d->c_elems, kEwiseN<T>);
+  switch (ceil_div(nvec, 256 * ceil_div(nvec, 4 * 256))) {
+    case 1: return launch_ewise_v<T, Ar, 1>(d, A, B, C, src, n_seg, stream);
+    case 2: return launch_ewise_v<T, Ar, 2>(d, A, B, C, src, n_seg, stream);
+    case 3: return launch_ewise_v<T, Ar, 3>(d, A, B, C, src, n_seg, stream);
+    default: return launch_ewise_v<T, Ar, 4>(d, A, B, C, src, n_seg, stream);
+  }
+}
+
+// Whether the einsum is an elementwise product of tiles of the same layout, of
+// one vector or more (smaller ones stay with the generic kernel: 400,000 pairs
+// of 6 bf16 elements in 13,000 segments 125 us, element by element here 149).
+bool is_ewise(const ej_einsum_desc *d, int32_t dtype) {
   if (d->a_elems != d->c_elems || d->b_elems != d->c_elems) return false;
+  if (d->c_elems < (dtype == EJ_BF16 ? 8 : 4)) return false;
   int64_t st = 1;
   for (int i = d->n_out - 1; i >= 0; --i) {
     if (d->out_ext[i] > 1 && (d->out_a[i] != st || d->out_b[i] != st)) return false;
@@ -2247,7 +2258,7 @@ bool try_stream(const ej_einsum_desc *d, int32_t dtype, const void *A, const voi
 
 int run_generic(const ej_einsum_desc *d, int32_t dtype, const void *A, const void *B, void *C,
                 const PairSrc &src, int64_t n_seg, hipStream_t stream) {
-  if (is_ewise(d) && n_seg < (int64_t(1) << 31) / ceil_div(d->c_elems, 4096)) {
+  if (is_ewise(d, dtype) && n_seg < (int64_t(1) << 31) / ceil_div(d->c_elems, 4096)) {
     if (dtype == EJ_I32) return launch_ewise<int32_t, GenInt32>(d, A, B, C, src, n_seg, stream);
     if (dtype == EJ_BF16) return launch_ewise<uint16_t, GenFloat>(d, A, B, C, src, n_seg, stream);
     return launch_ewise<float, GenFloat>(d, A, B, C, src, n_seg, stream);

@@ -555,6 +555,44 @@ def test_elementwise_tiles(gpu, tile, dtype):
         assert torch.equal(got, f32.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 7, 8, 9, 15, 17, 255, 257, 1023, 1024, 1025, 1028, 2047,
+                               2048, 2049, 4097, 8200])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32])
+def test_elementwise_tile_edges(gpu, n, dtype):
+    """Tiles below one 16-byte vector, a vector and its neighbours (the last
+    one moved back), 256 vectors and one more, several workgroups."""
+    test_elementwise_tiles(gpu, (n,), dtype)
+
+
+def _time_us(f, n=20):
+    for _ in range(3):
+        f()
+    ts = []
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(n):
+            f()
+        b.record()
+        torch.cuda.synchronize()
+        ts.append(a.elapsed_time(b) * 1e3 / n)
+    return sorted(ts)[2]
+
+
+@pytest.mark.parametrize("tile", [(4, 4), (16, 16), (20, 25)])
+def test_small_elementwise_tiles_are_no_slower(gpu, tile):
+    """Small tiles are no slower by vectors than element by element (the same
+    product stored transposed, which the general kernel takes): measured at
+    half its time; the bound leaves room for noise."""
+    note("small elementwise tiles", tile)
+    rng = np.random.default_rng(1)
+    a, b = (torch.randn((256, *tile), device="cuda").bfloat16() for _ in range(2))
+    idx = [torch.from_numpy(rng.integers(0, 256, 20000)).cuda() for _ in range(2)]
+    t = [_time_us(lambda d=_device.describe(s, tile, tile): _device.pair_einsum(d, a, b, *idx))
+         for s in ("ij,ij->ij", "ij,ij->ji")]
+    assert t[0] <= 1.3 * t[1], t
+
+
 @pytest.mark.parametrize("case", ["uniform", "skewed", "empty", "unsorted"])
 def test_first_call_queues_row_plan(gpu, case, monkeypatch):
     """The first call on relations made anew takes a guessed pair bound: enough, too
