@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
 
 # m, k, n: fragment edges (16), block edges (5 fragments), K blocks of 16 (fp32)
 # and 32 (bf16) with their tails, single rows and columns, several blocks.
-SIZES = [(1, 8, 1), (16, 16, 16), (17, 15, 33), (33, 31, 17), (48, 33, 49), (75, 75, 75),
+SIZES = [(1, 8, 1), (90, 33, 1), (16, 16, 16), (17, 15, 33), (33, 31, 17), (48, 33, 49), (75, 75, 75),
          (80, 80, 81), (81, 47, 80), (5, 100, 64), (64, 9, 1), (100, 20, 125), (161, 24, 97)]
 SPECS = {"ij,jk->ik": ("mk", "kn"), "ij,kj->ik": ("mk", "nk"), "ji,jk->ik": ("km", "kn"),
          "ji,kj->ik": ("km", "nk"), "ij,jk->ki": ("mk", "kn")}
