@@ -2366,19 +2366,17 @@ bool try_gemm(const ej_einsum_desc *d, int32_t dtype, const void *A, const void 
   }
   // fp32, K a multiple of 32, 16-byte rows, at least one operand in the layout
   // the forward has: the LDS-ring kernel with fp32 MFMAs (the forward's layout
-  // grouped like the bf16 one).
-  if (dtype == EJ_F32 && (ad || !bd) && d->k % 32 == 0 &&
-      (bm == 32 || bm == 64 || bm == 128) && src.n_a_tiles < (int64_t(1) << 31) &&
-      src.n_b_tiles < (int64_t(1) << 31)) {
-    const int fbn = d->n % 64 == 0 ? 64 : 32;
-    if (d->n % fbn == 0) {
-      g.nblocks = d->n / fbn;
-      const bool grouped = src.seg_off && d->seg_group > 0 && d->seg_group % 4 == 0;
-      *status = !ad  ? launch_seg_gemm_f32_t<true, false>(bm, fbn, A, B, C, src, g, n_seg, stream)
-                : bd ? launch_seg_gemm_f32_t<false, true>(bm, fbn, A, B, C, src, g, n_seg, stream)
-                     : launch_seg_gemm_f32(bm, fbn, grouped ? 4 : 1, A, B, C, src, g, n_seg, stream);
-      return true;
-    }
+  // grouped like the bf16 one).  Its tile indices are 31-bit; relations said to
+  // hold more tiles go to the generic kernel.
+  if (dtype == EJ_F32 && (ad || !bd) && bk == 32) {
+    if (src.n_a_tiles >= (int64_t(1) << 31) || src.n_b_tiles >= (int64_t(1) << 31)) return false;
+    const int fbn = bn >= 64 ? 64 : 32;
+    g.nblocks = d->n / fbn;
+    const bool grouped = src.seg_off && d->seg_group > 0 && d->seg_group % 4 == 0;
+    *status = !ad  ? launch_seg_gemm_f32_t<true, false>(bm, fbn, A, B, C, src, g, n_seg, stream)
+              : bd ? launch_seg_gemm_f32_t<false, true>(bm, fbn, A, B, C, src, g, n_seg, stream)
+                   : launch_seg_gemm_f32(bm, fbn, grouped ? 4 : 1, A, B, C, src, g, n_seg, stream);
+    return true;
   }
   if (dtype == EJ_BF16) {
     // 32-deep K stages for bf16 too: 32 KB of LDS, so three workgroups share

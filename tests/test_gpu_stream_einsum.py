@@ -363,3 +363,30 @@ def test_fp32_ring_transposed_layouts(gpu, spec, m, k, n):
         got = _run(spec, lt, rt, lv, rv, li, ri, perm, off, torch.float32)
         longest = int(np.diff(off).max()) * k
         assert R.rel_l2(got.cpu().numpy(), want) <= _tol(torch.float32, torch.float32, longest)
+
+
+@pytest.mark.parametrize("spec,lt,rt", [("ij,jk->ik", (64, 32), (32, 64)),
+                                        ("ij,kj->ik", (32, 64), (64, 64)),
+                                        ("ji,jk->ik", (32, 128), (32, 32)),
+                                        ("ji,kj->ik", (32, 32), (32, 32)),
+                                        ("ij,jk->ik", (20, 20), (20, 20)),
+                                        ("ij,ij->ij", (8, 8), (8, 8))])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_tile_counts_beyond_31_bits(gpu, spec, lt, rt, dtype):
+    """Relations said to hold 2^31 tiles (the pairs name the first few) are
+    taken, by the kernels whose tile indices are 64-bit."""
+    print("[case] tile counts", spec, lt, rt, dtype, flush=True)
+    rng = np.random.default_rng(4)
+    lv, rv = (R.bf16_round(rng.standard_normal((5, *t)).astype(np.float32)) for t in (lt, rt))
+    li, ri = rng.integers(0, 5, 12), rng.integers(0, 5, 12)
+    dev = lambda a: torch.from_numpy(a).cuda()
+    a, b, dli, dri = dev(lv).to(dtype), dev(rv).to(dtype), dev(li), dev(ri)
+    desc = _device.describe(spec, lt, rt)
+    desc.out_dtype = _lib.EJ_F32
+    want = R.kernel_einsum(lv, rv, li, ri, spec, precision="fp64")
+    out = torch.empty(want.shape, device="cuda")
+    assert _lib.load().ej_pair_einsum(
+        ctypes.byref(desc), _lib.EJ_BF16 if dtype == torch.bfloat16 else _lib.EJ_F32,
+        _device.ptr(a), _device.ptr(b), 1 << 31, 1 << 31, _device.ptr(dli), _device.ptr(dri), 12,
+        _device.ptr(out), _device.stream_ptr()) == _lib.EJ_OK
+    assert R.rel_l2(out.cpu().numpy(), want) <= _tol(dtype, torch.float32, max(desc.k, 1))
