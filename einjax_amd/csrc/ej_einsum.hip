@@ -2393,7 +2393,7 @@ bool try_gemm(const ej_einsum_desc *d, int32_t dtype, const void *A, const void 
 // The streaming GEMM for the GEMM-shaped einsums that the blocked kernels do
 // not take (extents that are no multiples of their blocks, rows that are not
 // 16-byte aligned): any extents and strides with at least one lane's k values
-// per row, tiles of less than 2 GB and 31-bit tile indices.  K below that
+// per row, tiles of less than 2 GB, 31-bit tile indices and 2^26 output blocks.  K below that
 // (outer and elementwise products) stays with the generic kernel: a K block
 // would be nearly all padding.
 bool try_stream(const ej_einsum_desc *d, int32_t dtype, const void *A, const void *B, void *C,
@@ -2408,7 +2408,6 @@ bool try_stream(const ej_einsum_desc *d, int32_t dtype, const void *A, const voi
   if (d->a_elems * esz >= lim || d->b_elems * esz >= lim || d->c_elems * 4 >= lim ||
       src.n_a_tiles >= lim || src.n_b_tiles >= lim || n_seg >= lim)
     return false;
-  if (n_seg * ceil_div(d->m, 16) * ceil_div(d->n, 16) * d->batch >= lim) return false;
   const int am = d->a_sk == 1 ? kStreamKC : d->a_sm == 1 ? kStreamFC : kStreamGS;
   // A single column is contiguous along n too, which spares a [k][m] lhs the
   // element loads (20,000 pairs of 'ij,i->j' on 128 x 128 fp32: 157 us, by
@@ -2417,6 +2416,12 @@ bool try_stream(const ej_einsum_desc *d, int32_t dtype, const void *A, const voi
                  : d->b_sk == 1               ? kStreamKC
                  : d->b_sn == 1               ? kStreamFC
                                               : kStreamGS;
+  // Output blocks of at most two or five fragments a side, each a quarter of a
+  // workgroup: a launch holds fewer than 2^32 threads.
+  const bool gs = am == kStreamGS || bm == kStreamGS || (am == kStreamFC && bm == kStreamKC);
+  const int64_t units = n_seg * d->batch * ceil_div(ceil_div(d->m, 16), gs ? 2 : 5) *
+                        ceil_div(ceil_div(d->n, 16), gs ? 2 : 5);
+  if (units >= (int64_t(1) << 26)) return false;
   GemmGeom g;
   g.m = d->m; g.n = d->n; g.k = d->k; g.batch = d->batch;
   g.a_sb = d->a_sb; g.a_sm = d->a_sm; g.a_sk = d->a_sk;

@@ -497,7 +497,7 @@ __global__ __launch_bounds__(256, stream_waves(FM * FN)) void stream_gemm_kernel
     const int64_t nl = ld_uniform(src.n_live, 0);
     nseg = nl < nseg ? nl : nseg;
   }
-  // below 2^31 (try_stream)
+  // below 2^26 (try_stream)
   const uint32_t units = static_cast<uint32_t>(nseg * (g.nblocks * g.mblocks * g.batch));
   if (units < kStreamSplitBlocks) {
     if (blockIdx.x >= units) return;
@@ -537,10 +537,6 @@ int launch_stream_t(const void *A, const void *B, void *C, const PairSrc &src, G
   const int64_t units = n_seg * g.mblocks * g.nblocks * g.batch;
   int64_t nblk = units < kStreamSplitBlocks ? units : ceil_div(units, 4);
   if (src.n_live && units >= kStreamSplitBlocks) nblk = std::max(nblk, kStreamSplitBlocks - 1);
-  if (units >= (int64_t(1) << 31)) {
-    set_error("einsum launch too large");
-    return EJ_E_UNSUPPORTED;
-  }
   hipLaunchKernelGGL((stream_gemm_kernel<T, FM, FN, AMODE, BMODE>),
                      dim3(static_cast<unsigned>(nblk)), dim3(256), 0, stream,
                      static_cast<const T *>(A), static_cast<const T *>(B), C, src, g, n_seg);

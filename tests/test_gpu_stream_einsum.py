@@ -390,3 +390,16 @@ def test_tile_counts_beyond_31_bits(gpu, spec, lt, rt, dtype):
         _device.ptr(a), _device.ptr(b), 1 << 31, 1 << 31, _device.ptr(dli), _device.ptr(dri), 12,
         _device.ptr(out), _device.stream_ptr()) == _lib.EJ_OK
     assert R.rel_l2(out.cpu().numpy(), want) <= _tol(dtype, torch.float32, max(desc.k, 1))
+
+
+@pytest.mark.parametrize("pairs", [(1 << 23) - 1, 1 << 23])
+def test_launches_near_their_limit(gpu, pairs):
+    """Row products of 33 outputs, eight lanes each: two workgroups a pair, of
+    which 2^24 are one too many for a launch; the generic kernel takes those."""
+    print("[case] launch limit", pairs, flush=True)
+    torch.manual_seed(0)
+    a, b = (torch.randint(-3, 4, (50, 33, 32), device="cuda").float() for _ in range(2))
+    li, ri = (torch.randint(0, 50, (pairs,), device="cuda") for _ in range(2))
+    got = _device.pair_einsum(_device.describe("ij,ij->i", (33, 32), (33, 32)), a, b, li, ri)
+    table = (a[:, None] * b[None]).sum(-1)  # small whole numbers: exact in any order
+    assert torch.equal(got, table[li, ri])
