@@ -127,6 +127,7 @@ class ExecutionEngine:
         else:
             self.mesh_axis_names = mesh_axis_names or ("x", "y", "z", "w")
         self.step_options = step_options
+        self._missed = {}  # steps whose guessed row plan missed: calls to go without one
 
     def _execute_einsum(self, formula: str, source_arrays: list, source_schemes=None,
                         output_scheme=None):
@@ -145,7 +146,7 @@ class ExecutionEngine:
                                       "engine runs steps whose operands are SparseTensorRelation")
         join, agg = relation_einsum_plan(formula, lhs.tile_shape, rhs.tile_shape)
         return execute_sparse(lhs, rhs, join, formula, agg,
-                              **{"_new_relations": True, **self.step_options})
+                              **{"_new_relations": self._missed, **self.step_options})
 
     def execute_plan(self, plan, operands: list, gather_output: bool = False):
         """Runs plan.steps in order over a working list that starts as the

@@ -427,6 +427,10 @@ def _dense_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, events):
     return None
 
 
+def _row_key(lhs, rhs, lc, rc, keys, agg):
+    return _hint_key(lhs, rhs, ("row", tuple(lc.shape), tuple(rc.shape), tuple(keys), tuple(agg)))
+
+
 def _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound, pair_key, events):
     """The whole step on the sorted row plan (three plan launches, then the
     fused einsum) when the join's structure suits it: (result, step,
@@ -441,8 +445,7 @@ def _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound, pair_key,
     rgrid = [_grid(rhs, d) for d in range(nr)]
     if not _device.row_plan_applies(lc.shape[0], lgrid, rgrid, keys, agg):
         return None
-    rkey = _hint_key(lhs, rhs, ("row", tuple(lc.shape), tuple(rc.shape), tuple(keys),
-                                tuple(agg)))
+    rkey = _row_key(lhs, rhs, lc, rc, keys, agg)
     if _hint_get(rkey, lhs, rhs) == -1:
         return None
     for _ in range(2):
@@ -463,6 +466,11 @@ def _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound, pair_key,
 # Output buffers of a guessed step hold at most this (larger einsums are not
 # bound by the waits the guess saves).
 _GUESS_MAX_BYTES = 256 << 20
+# A guess that misses (unsorted relations, more pairs than the row plan counts)
+# costs 85 us beside a call of 220; an engine tries such a step again after this
+# many calls, for at most _MISSED_MAX steps.
+_MISS_SKIP = 32
+_MISSED_MAX = 256
 
 
 def _pair_guess(lhs, rhs, keys, kernel_string, nl: int, nr: int, out_dtype):
@@ -808,7 +816,7 @@ def _empty_result(lhs, n_out, out_tile, output_shape, host, out_dtype=None):
 def execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_keys,
                    kernel_string: str, agg_keys, output_shape=None, output_tile_shape=None, *,
                    fused: bool = True, out_dtype=None,
-                   _einsum_events=None, _new_relations: bool = False) -> SparseTensorRelation:
+                   _einsum_events=None, _new_relations=False) -> SparseTensorRelation:
     try:
         return _execute_sparse(lhs, rhs, join_keys, kernel_string, agg_keys, output_shape,
                                output_tile_shape, fused=fused, out_dtype=out_dtype,
@@ -845,7 +853,7 @@ def execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_ke
 def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_keys,
                     kernel_string: str, agg_keys, output_shape=None, output_tile_shape=None, *,
                     fused: bool = True, out_dtype=None,
-                    _einsum_events=None, _new_relations: bool = False) -> SparseTensorRelation:
+                    _einsum_events=None, _new_relations=False) -> SparseTensorRelation:
     """Sparse tensor-relational einsum (reference: sparse_dispatch.py:226-297).
 
     join_keys: [(lhs_dim, rhs_dim)] contracted tile dims; kernel_string: the
@@ -862,7 +870,8 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
     only): a list that collects timing events recorded around the fused
     einsum of a queued call.  ``_new_relations`` (the engine's steps): the
     relations are made anew for each call, so a first call is queued on a
-    guessed pair bound (_pair_guess).  Integer or boolean tiles (and a float with an
+    guessed pair bound (_pair_guess); a dict counts down the calls, per kind of
+    step, that go without a guess after one that missed.  Integer or boolean tiles (and a float with an
     integer) follow the reference's jnp promotion (kernel_einsum) and run on
     the library's integer kernel; joined and output coordinates may be
     negative."""
@@ -940,9 +949,16 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
         hint_key = _hint_key(lhs, rhs, (tuple(lc.shape), tuple(rc.shape), tuple(keys),
                                         tuple(j_rad), tuple(agg)))
         bound = _hint_get(hint_key, lhs, rhs)
-        if bound is None and _new_relations:
-            guess = _pair_guess(lhs, rhs, keys, kernel_string, lc.shape[0], rc.shape[0],
-                                out_dtype)
+        if bound is None and _new_relations is not False:
+            call = (kernel_string, tuple(lhs.shape), tuple(lhs.tile_shape), tuple(rhs.shape),
+                    tuple(rhs.tile_shape), tuple(keys), tuple(agg))
+            missed = _new_relations if isinstance(_new_relations, dict) else {}
+            skip = missed.get(call, 0)
+            if skip:
+                missed[call] = skip - 1
+            else:
+                guess = _pair_guess(lhs, rhs, keys, kernel_string, lc.shape[0], rc.shape[0],
+                                    out_dtype)
         if (bound or guess or 0) > 0:
             done = _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound or guess,
                              hint_key, _einsum_events)
@@ -951,6 +967,11 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
                 kind, dkey = "row", (hint_key, rkey)
             else:
                 bound = _hint_get(hint_key, lhs, rhs)
+                if guess is not None and _hint_get(_row_key(lhs, rhs, lc, rc, keys, agg), lhs,
+                                                   rhs) == -1:
+                    if len(missed) >= _MISSED_MAX:
+                        missed.clear()
+                    missed[call] = _MISS_SKIP
         if queued is None and bound is not None and bound > 0:
             desc, a, b = operands()
             step = _device.QueuedStep(lc, rc, keys, j_rad, agg, radices(None), desc, a, b,

@@ -22,6 +22,7 @@ from oracle import reference_path as R
 import einjax_amd as ej
 from einjax_amd import SparseTensorRelation, _device, _lib
 from einjax_amd.execution import sparse_dispatch as sd
+from einjax_amd.execution.engine import ContractionPlan, ContractionStep
 
 pytestmark = pytest.mark.gpu
 
@@ -631,3 +632,35 @@ def test_first_call_queues_row_plan(gpu, case, monkeypatch):
     sd._pair_hints.clear()
     want = ej.execute_sparse(L, Rr, *args)
     assert torch.equal(got.coords, want.coords) and torch.equal(got.values, want.values)
+
+
+def test_engine_seldom_repeats_a_missed_guess(gpu, monkeypatch):
+    """Steps on new relations that do not suit the row plan (unsorted tiles)
+    try it once, then take the general plan at once for a number of calls; a
+    step on other grids still tries it."""
+    note("engine miss")
+    rng = np.random.default_rng(3)
+    a, b = sparse_rel(rng, (24, 40), (32, 32), 0.2), sparse_rel(rng, (40, 16), (32, 32), 0.2)
+    p = rng.permutation(len(a.coords))
+    a = R.Rel(a.coords[p], a.values[p], a.shape, a.tile_shape)
+    statuses = []
+    run = _device.run_row_step
+
+    def spy(step, events=None):
+        r = run(step, events)
+        statuses.append(r[0])
+        return r
+
+    monkeypatch.setattr(_device, "run_row_step", spy)
+    monkeypatch.setattr(sd, "_MISS_SKIP", 3)
+    plan = ContractionPlan("ij,jk->ik", [ContractionStep(0, "ij,jk->ik", (0, 1))])
+    engine = ej.ExecutionEngine()
+    want = R.execute_sparse(a, b, [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)], precision="fp64")
+    for call in range(6):
+        got = engine.execute_plan(plan, [dev_rel(a), dev_rel(b)])
+        npt.assert_array_equal(got.coords.cpu().numpy(), want.coords)
+        assert R.rel_l2(got.values.cpu().numpy(), want.values) <= 1e-5
+        assert statuses == ["miss"] * (1 if call < 4 else 2)
+    c = sparse_rel(rng, (24, 30), (32, 32), 0.2), sparse_rel(rng, (30, 16), (32, 32), 0.2)
+    engine.execute_plan(plan, [dev_rel(x) for x in c])
+    assert statuses == ["miss", "miss", "ok"]
