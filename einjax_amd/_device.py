@@ -589,6 +589,7 @@ def run_dense_step(step: DenseStep, einsum_events=None):
 # Limits of ej_row_plan_async (the library refuses beyond them).
 ROW_MAX_LHS, ROW_MAX_JOIN, ROW_MAX_FREE, ROW_MAX_RUNS = 16384, 65536, 8192, 8192
 _ROW_COUNT_MASK = (1 << 21) - 1
+ROW_MAX_PAIRS = _ROW_COUNT_MASK  # counts from here on are a miss (run_row_step)
 
 
 def row_plan_applies(n_lhs: int, lhs_grid, rhs_grid, join_keys, agg_keys) -> bool:

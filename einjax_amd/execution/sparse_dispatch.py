@@ -463,8 +463,8 @@ def _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound, pair_key,
     return None
 
 
-# Output buffers of a guessed step hold at most this (larger einsums are not
-# bound by the waits the guess saves).
+# A guessed step's buffers (outputs, pair indices, offsets and coordinates) hold
+# at most this (larger einsums are not bound by the waits the guess saves).
 _GUESS_MAX_BYTES = 256 << 20
 # A guess that misses (unsorted relations, more pairs than the row plan counts)
 # costs 85 us beside a call of 220; an engine tries such a step again after this
@@ -473,15 +473,15 @@ _MISS_SKIP = 32
 _MISSED_MAX = 256
 
 
-def _pair_guess(lhs, rhs, keys, kernel_string, nl: int, nr: int, out_dtype):
+def _pair_guess(lhs, rhs, keys, agg, kernel_string, nl: int, nr: int, out_dtype):
     """A pair bound for the first call on two relations, for callers that seldom
     make a second one, so that it too can queue the row plan and the einsum
     without waiting for a count: the pairs of uniformly spread tiles and a
     quarter more.  A guess that is too small
     is detected on the device and costs one more plan with the exact count.
-    None where the general plan is to answer: large outputs, a stream under
-    capture (the count's wait would not end), or a call the library would
-    refuse only once there are pairs.
+    None where the general plan is to answer: large buffers, more pairs than
+    the row plan counts, a stream under capture (the count's wait would not
+    end), or a call the library would refuse only once there are pairs.
     A three-operand chain on 32 x 32 fp32 tiles, whose second step always
     meets a new relation: 302 us a call with the general plan and its
     host waits, 179-188 us so."""
@@ -497,7 +497,10 @@ def _pair_guess(lhs, rhs, keys, kernel_string, nl: int, nr: int, out_dtype):
         elems = _device.describe(kernel_string, lhs.tile_shape, rhs.tile_shape).c_elems
     except (ValueError, TypeError, RuntimeError):
         return None
-    return guess if 4 * elems * guess <= _GUESS_MAX_BYTES else None
+    per_pair = 4 * elems + 16 + 4 + 4 * len(agg)
+    if guess >= _device.ROW_MAX_PAIRS or per_pair * guess > _GUESS_MAX_BYTES:
+        return None
+    return guess
 
 
 # ---------------------------------------------------------------------------
@@ -957,8 +960,8 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
             if skip:
                 missed[call] = skip - 1
             else:
-                guess = _pair_guess(lhs, rhs, keys, kernel_string, lc.shape[0], rc.shape[0],
-                                    out_dtype)
+                guess = _pair_guess(lhs, rhs, keys, agg, kernel_string, lc.shape[0],
+                                    rc.shape[0], out_dtype)
         if (bound or guess or 0) > 0:
             done = _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound or guess,
                              hint_key, _einsum_events)

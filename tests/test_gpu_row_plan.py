@@ -664,3 +664,22 @@ def test_engine_seldom_repeats_a_missed_guess(gpu, monkeypatch):
     c = sparse_rel(rng, (24, 30), (32, 32), 0.2), sparse_rel(rng, (30, 16), (32, 32), 0.2)
     engine.execute_plan(plan, [dev_rel(x) for x in c])
     assert statuses == ["miss", "miss", "ok"]
+
+
+@pytest.mark.parametrize("tile,side,guessed", [((64, 64), 60, True), ((64, 64), 300, False),
+                                               ((1, 1), 1000, True), ((1, 1), 2700, False)])
+def test_guessed_bounds_stay_within_limits(gpu, tile, side, guessed, monkeypatch):
+    """No guess beyond what the row plan counts or a quarter gigabyte for
+    outputs, pairs and plan: 1 x 1 tiles are limited by the counts, their
+    outputs being small."""
+    note("guess limits", tile, side)
+    c = torch.stack([torch.arange(side, dtype=torch.int32), torch.zeros(side, dtype=torch.int32)], 1)
+    shape = (side * tile[0], 4 * tile[1])  # one of four join indices is there
+    L = SparseTensorRelation(c.cuda(), torch.ones((side, *tile), device="cuda"), shape, tile)
+    Rr = SparseTensorRelation(c.flip(1).contiguous().cuda(), L.values, shape[::-1], tile)
+    guesses = []
+    real = sd._pair_guess
+    monkeypatch.setattr(sd, "_pair_guess", lambda *a: guesses.append(real(*a)) or guesses[-1])
+    got = ej.execute_sparse(L, Rr, [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)], _new_relations=True)
+    assert [g is not None for g in guesses] == [guessed]
+    assert got.coords.shape[0] == side * side and bool((got.values == tile[1]).all())
