@@ -503,6 +503,11 @@ def _pair_guess(lhs, rhs, keys, agg, kernel_string, nl: int, nr: int, out_dtype)
     return guess
 
 
+# A guessed step's result is copied out of buffers of more than twice its size
+# (and this much more): the relation would keep all of them alive.
+_GUESS_SPARE_BYTES = 1 << 20
+
+
 # ---------------------------------------------------------------------------
 # Repeated calls.  A queued step on device relations keeps its prepared plan
 # and einsum (a DenseStep or QueuedStep: argument lists, capacities, output
@@ -937,6 +942,11 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
         return out
 
     keys = [tuple(k) for k in join_keys]
+
+    def call():  # the kind of step, for an engine's misses
+        return (kernel_string, tuple(lhs.shape), tuple(lhs.tile_shape), tuple(rhs.shape),
+                tuple(rhs.tile_shape), tuple(keys), tuple(agg))
+
     hint_key = None
     bound = None
     queued = guess = None
@@ -953,12 +963,10 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
                                         tuple(j_rad), tuple(agg)))
         bound = _hint_get(hint_key, lhs, rhs)
         if bound is None and _new_relations is not False:
-            call = (kernel_string, tuple(lhs.shape), tuple(lhs.tile_shape), tuple(rhs.shape),
-                    tuple(rhs.tile_shape), tuple(keys), tuple(agg))
             missed = _new_relations if isinstance(_new_relations, dict) else {}
-            skip = missed.get(call, 0)
+            skip = missed.get(call(), 0) if missed else 0
             if skip:
-                missed[call] = skip - 1
+                missed[call()] = skip - 1
             else:
                 guess = _pair_guess(lhs, rhs, keys, agg, kernel_string, lc.shape[0],
                                     rc.shape[0], out_dtype)
@@ -974,7 +982,7 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
                                                    rhs) == -1:
                     if len(missed) >= _MISSED_MAX:
                         missed.clear()
-                    missed[call] = _MISS_SKIP
+                    missed[call()] = _MISS_SKIP
         if queued is None and bound is not None and bound > 0:
             desc, a, b = operands()
             step = _device.QueuedStep(lc, rc, keys, j_rad, agg, radices(None), desc, a, b,
@@ -995,7 +1003,12 @@ def _execute_sparse(lhs: SparseTensorRelation, rhs: SparseTensorRelation, join_k
             _remember_step(step_key, lhs, rhs, kind, step, dkey, fin)
         if P == 0:
             return _empty_result(lhs, n_out, output_tile_shape, output_shape, host, out_dtype)
+        spare = step.cap_u - U
         coords, vals = coords[:U], vals[:U]
+        if guess is not None and spare > U:
+            coords, vals = (
+                t.clone() if spare * t.stride(0) * t.element_size() > _GUESS_SPARE_BYTES else t
+                for t in (coords, vals))
     else:
         li, ri = _join_dev(lhs, rhs, join_keys, lc, rc)
         if hint_key is not None and (bound is None or bound >= 0):

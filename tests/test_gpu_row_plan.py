@@ -683,3 +683,25 @@ def test_guessed_bounds_stay_within_limits(gpu, tile, side, guessed, monkeypatch
     got = ej.execute_sparse(L, Rr, [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)], _new_relations=True)
     assert [g is not None for g in guesses] == [guessed]
     assert got.coords.shape[0] == side * side and bool((got.values == tile[1]).all())
+
+
+def test_guessed_results_do_not_keep_their_buffers(gpu):
+    """A join of few output tiles from many pairs on a large grid: the guess
+    sizes buffers for most of the pairs, the result keeps its own size."""
+    note("guessed result's size")
+    tile = (32, 32)
+    i, j = np.meshgrid(np.arange(3), np.arange(400), indexing="ij")
+    ca = np.stack([i.ravel(), j.ravel()], 1).astype(np.int32)
+    cb = np.stack([j.T.ravel(), i.T.ravel()], 1).astype(np.int32)
+    rng = np.random.default_rng(2)
+    shape = (100 * 32, 400 * 32)
+    a, b = (R.Rel(c, rng.standard_normal((len(c), *tile)).astype(np.float32), s, tile)
+            for c, s in ((ca, shape), (cb, shape[::-1])))
+    got = ej.execute_sparse(dev_rel(a), dev_rel(b), [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)],
+                            _new_relations=True)
+    assert got.coords.shape[0] == 9
+    for t in (got.coords, got.values):
+        assert t.untyped_storage().nbytes() <= 2 * t.numel() * t.element_size() + (1 << 20)
+    want = R.execute_sparse(a, b, [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)], precision="fp64")
+    npt.assert_array_equal(got.coords.cpu().numpy(), want.coords)
+    assert R.rel_l2(got.values.cpu().numpy(), want.values) <= 1e-5
