@@ -700,8 +700,9 @@ def test_guessed_results_do_not_keep_their_buffers(gpu):
     got = ej.execute_sparse(dev_rel(a), dev_rel(b), [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)],
                             _new_relations=True)
     assert got.coords.shape[0] == 9
-    for t in (got.coords, got.values):
-        assert t.untyped_storage().nbytes() <= 2 * t.numel() * t.element_size() + (1 << 20)
+    for t in (got.coords, got.values):  # (plain numbers: a storage prints element by element)
+        held, used = int(t.untyped_storage().nbytes()), t.numel() * t.element_size()
+        assert held <= 2 * used + (1 << 20)
     want = R.execute_sparse(a, b, [(1, 0)], "ij,jk->ik", [(0, 0), (1, 1)], precision="fp64")
     npt.assert_array_equal(got.coords.cpu().numpy(), want.coords)
     assert R.rel_l2(got.values.cpu().numpy(), want.values) <= 1e-5
