@@ -2157,14 +2157,17 @@ SegSplit seg_split(int G, int64_t n_seg, int64_t batch, int64_t nblocks, int64_t
   return r;
 }
 
-template <class Op, int G, int WGM, int NW, int NSW = EJ_SEG_NS, bool LINES = false>
+template <class Op, int G, int WGM, int NW, int NSW = EJ_SEG_NS, bool LINES = false,
+          bool MULTI = true>
 int launch_seg_gemm_t(const void *A, const void *B, void *C, const PairSrc &src_in,
                       const GemmGeom &g, int64_t n_seg, hipStream_t stream) {
   constexpr int NS = seg_ring_depth(Op::A_BYTES + G * Op::B_BYTES, NSW);
   PairSrc src = src_in;
   if (src.order_group != G) src.run_order = nullptr;  // an order for other groups
   const int64_t groups = ceil_div(n_seg, G);
-  const SegSplit sp = seg_split(G, n_seg, g.batch, g.nblocks, g.mblocks, src.seg_off != nullptr);
+  SegSplit sp{0, 1, g.batch * g.nblocks * g.mblocks};  // one block of one group a workgroup
+  if constexpr (MULTI)
+    sp = seg_split(G, n_seg, g.batch, g.nblocks, g.mblocks, src.seg_off != nullptr);
   const int mb_loop = sp.mb_loop, spw = sp.spw;
   const int64_t per_group = sp.per_group;
   const int64_t nblk = ceil_div(groups, spw) * per_group;
@@ -2174,16 +2177,18 @@ int launch_seg_gemm_t(const void *A, const void *B, void *C, const PairSrc &src_
   }
   using TA = typename Op::a_elem;
   using TB = typename Op::b_elem;
-  if (mb_loop || spw > 1)
-    hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, true, LINES>),
-                       dim3(static_cast<unsigned>(nblk)), dim3(NW * 64), 0, stream,
-                       static_cast<const TA *>(A), static_cast<const TB *>(B), C, src, g, n_seg,
-                       spw, mb_loop);
-  else
-    hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, false, LINES>),
-                       dim3(static_cast<unsigned>(nblk)), dim3(NW * 64), 0, stream,
-                       static_cast<const TA *>(A), static_cast<const TB *>(B), C, src, g, n_seg, 1,
-                       0);
+  if constexpr (MULTI)
+    if (sp.multi()) {
+      hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, true, LINES>),
+                         dim3(static_cast<unsigned>(nblk)), dim3(NW * 64), 0, stream,
+                         static_cast<const TA *>(A), static_cast<const TB *>(B), C, src, g, n_seg,
+                         spw, mb_loop);
+      EJ_LAUNCH_CHECK();
+      return EJ_OK;
+    }
+  hipLaunchKernelGGL((seg_gemm_kernel<Op, NS, G, WGM, NW, false, LINES>),
+                     dim3(static_cast<unsigned>(nblk)), dim3(NW * 64), 0, stream,
+                     static_cast<const TA *>(A), static_cast<const TB *>(B), C, src, g, n_seg, 1, 0);
   EJ_LAUNCH_CHECK();
   return EJ_OK;
 }
@@ -2240,14 +2245,18 @@ int launch_seg_gemm_f32(int bm, int bn, int grp, const void *A, const void *B, v
 }
 
 // The same with an [n][k] rhs (AT = false, BT = true) or a [k][m] lhs (AT =
-// true, BT = false), one segment per workgroup.
+// true, BT = false), one block of one segment per workgroup.  Workgroups that
+// walk several blocks or segments leave the chip too few of them at a time: both
+// gradients of 10,496 pairs of 96 x 96 x 96 (3 x 3 blocks of 32) 290 + 493 us so,
+// 248 + 262 us one block each (register-staged kernel 288 + 338).
 template <bool AT, bool BT>
 int launch_seg_gemm_f32_t(int bm, int bn, const void *A, const void *B, void *C,
                           const PairSrc &src, const GemmGeom &g, int64_t n_seg,
                           hipStream_t stream) {
-#define EJ_F32_CASE(M_, N_, WGM_)  \
-  if (bm == M_ && bn == N_)        \
-    return launch_seg_gemm_t<SegOpF32<M_, N_, AT, BT>, 1, WGM_, 4>(A, B, C, src, g, n_seg, stream);
+#define EJ_F32_CASE(M_, N_, WGM_)                                                              \
+  if (bm == M_ && bn == N_)                                                                    \
+    return launch_seg_gemm_t<SegOpF32<M_, N_, AT, BT>, 1, WGM_, 4, EJ_SEG_NS, false, false>(     \
+        A, B, C, src, g, n_seg, stream);
   EJ_F32_CASE(32, 32, 2) EJ_F32_CASE(32, 64, 2) EJ_F32_CASE(64, 32, 2)
   EJ_F32_CASE(64, 64, 2) EJ_F32_CASE(128, 32, 4) EJ_F32_CASE(128, 64, 2)
 #undef EJ_F32_CASE
