@@ -255,6 +255,18 @@ VecRows vec_rows(const BucketGeom &g, int esz) {
   return v;
 }
 
+// Whether the tiles of a dense tensor are cut by vectors.  Two float64 elements
+// a vector do not pay for rows off 16 bytes, where element loads are already
+// half as wide (4000^2 in tiles of 80 x 25: 112 us by vectors, 99 by elements;
+// rank 3, whose elements each take a decoded row, 96 by vectors, 105).  Nor do
+// overlapping vectors in tiles of a few (3969^2 in tiles of 9 x 9: 500 us, 481).
+bool cut_by_vectors(const BucketGeom &g, const VecRows &v, int esz, const void *dense) {
+  if (v.n == 0 || (v.n < 32 && g.inner * esz % 16 != 0)) return false;
+  if (esz != 8 || g.nd != 2) return true;
+  return ((reinterpret_cast<uintptr_t>(dense) | static_cast<uintptr_t>(v.pitch) |
+           static_cast<uintptr_t>(g.inner * esz)) & 15) == 0;
+}
+
 __global__ void slot_map_kernel(const int64_t *flags, const int64_t *excl, int64_t n,
                                 int64_t *tile_of_slot) {
   int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -403,7 +415,7 @@ extern "C" int ej_bucket_dense_count(const void *dense, int32_t dtype, int32_t n
   const VecRows v = vec_rows(g, esz);
   const dim3 grid(static_cast<unsigned>(g.n_tiles));
   const unsigned char *db = static_cast<const unsigned char *>(dense);
-  if (v.n > 0) {
+  if (cut_by_vectors(g, v, esz, dense)) {
 #define EJ_FLAGS(M, N2) hipLaunchKernelGGL((tile_flags_vec_kernel<M, N2>), grid, dim3(256), 0, stream, db, g, v, w.flags)
     if (g.nd == 2) {
       if (mode == 0) EJ_FLAGS(0, true); else if (mode == 1) EJ_FLAGS(1, true); else EJ_FLAGS(2, true);
@@ -455,7 +467,7 @@ extern "C" int ej_bucket_dense_fill(const void *dense, int32_t dtype, int32_t nd
   const int mode = dtype == EJ_F64 ? 2 : dtype == EJ_F32 ? 1 : 0;
   const VecRows v = vec_rows(g, esz);
   const dim3 grid(static_cast<unsigned>(n_tiles));
-  if (v.n > 0) {
+  if (cut_by_vectors(g, v, esz, dense)) {
     const unsigned char *db = static_cast<const unsigned char *>(dense);
     unsigned char *vb = static_cast<unsigned char *>(values);
 #define EJ_COPY(M, N2) hipLaunchKernelGGL((tile_copy_vec_kernel<M, N2>), grid, dim3(256), 0, stream, db, g, v, w.tile_of_slot, w.scalars, coords, vb)
@@ -508,8 +520,10 @@ extern "C" int ej_relation_to_dense(const int32_t *coords, const void *values, i
   EJ_LAUNCH_CHECK();
   if (n_tiles == 0) return EJ_OK;
   EJ_CHECK_ARG(coords && values, "null pointer argument");
+  // Tiles of up to 16 vectors are bound by the number of workgroups (2^19 tiles of
+  // 8 elements: 225 us by elements, 240 by vectors).
   const VecRows v = vec_rows(g, dtype == EJ_F64 ? 8 : dtype == EJ_F32 ? 4 : 2);
-  if (v.n > 0) {
+  if (v.n > 16) {
     const unsigned char *vb = static_cast<const unsigned char *>(values);
     unsigned char *db = static_cast<unsigned char *>(dense);
 #define EJ_SCATTER(E, N2) hipLaunchKernelGGL((scatter_tiles_vec_kernel<E, N2>), dim3(static_cast<unsigned>(n_tiles)), dim3(256), 0, stream, coords, vb, g, v, db)
