@@ -2345,8 +2345,12 @@ bool try_gemm(const ej_einsum_desc *d, int32_t dtype, const void *A, const void 
     // alone take 51 us, stores alone 121, loads and MFMAs alone 178). Measured
     // against tile_gemm_dma_kernel: those pairs 303 / 357 us, 13,107 pairs of
     // 64 x 64 x 64 42 / 71 us. With segments the two are within 10% of each
-    // other either way, so those keep the 64-deep kernel below.
-    if (!src.seg_off && ad && !bd) {
+    // other either way, so those keep the 64-deep kernel below.  So do long
+    // contractions of fewer pairs than the chip holds workgroups, bound by the
+    // latency of the stages (100 pairs of 128 x 512 x 128: 13.4 / 15.8 us; both
+    // kernels add in the same order).
+    const bool few = d->k % 64 == 0 && d->k >= 512 && nblk < 512;
+    if (!src.seg_off && ad && !bd && !few) {
       *status = bm == 128
                     ? launch_seg_gemm_t<SegOpBf16<128, 128>, 1, 2, 4, EJ_SEG_NS, true>(
                           A, B, C, src, g, n_seg, stream)

@@ -342,6 +342,24 @@ def test_pair_results_in_lines(gpu, m, k, n, spec):
     assert torch.equal(flat[1:].view(got.shape), got)
 
 
+@pytest.mark.parametrize("m,n", [(64, 64), (128, 128), (128, 256)])
+@pytest.mark.parametrize("k", [448, 512, 576])
+def test_pair_results_of_few_long_products(gpu, m, n, k):
+    """Per-pair bf16 products of a long contraction, few of them (deep stages)
+    and many (the ring): the same bits, and float64 within rounding."""
+    print("[case] few long pairs", m, n, k, flush=True)
+    lt, rt, lv, rv, li, ri, _, _ = _case("ij,jk->ik", m, k, n, torch.bfloat16, k, pairs=600)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    a, b, li_, ri_ = dev(lv).bfloat16(), dev(rv).bfloat16(), dev(li), dev(ri)
+    desc = _device.describe("ij,jk->ik", lt, rt)
+    for out in (torch.float32, torch.bfloat16):
+        many = _device.pair_einsum(desc, a, b, li_, ri_, out_dtype=out)
+        few = _device.pair_einsum(desc, a, b, li_[:40], ri_[:40], out_dtype=out)
+        assert torch.equal(many[:40], few)
+        want = R.kernel_einsum(lv, rv, li[:40], ri[:40], "ij,jk->ik", precision="fp64")
+        assert R.rel_l2(few.float().cpu().numpy(), want) <= _tol(torch.bfloat16, out, k)
+
+
 @pytest.mark.parametrize("spec", ["ij,kj->ik", "ji,jk->ik"])
 @pytest.mark.parametrize("m,k,n", [(32, 32, 32), (64, 64, 64), (128, 32, 128), (96, 160, 32),
                                    (32, 64, 192), (192, 96, 96)])
