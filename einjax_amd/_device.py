@@ -658,8 +658,8 @@ class RowStep:
 
 
 def run_row_step(step: RowStep, einsum_events=None):
-    """Queues one call of a prepared RowStep: the three-launch row plan and
-    the fused segment einsum back to back on the current stream, then waits
+    """Queues one call of a prepared RowStep: the row plan (three launches, two
+    where tile meets tile) and the fused segment einsum back to back on the current stream, then waits
     for the plan's packed count word.  Returns (status, result): "ok" with
     result = (P, U, coords [cap_u, n_out], values [cap_u, *out_tile],
     workspace) (the first U rows of coords and values are the output);

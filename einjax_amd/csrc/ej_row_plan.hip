@@ -1,5 +1,6 @@
 // Join and segment plan of a sparse einsum whose operands are both sorted
-// relations, row by row, in three launches and without sorting.
+// relations, row by row, in three launches (two where tile meets tile) and without
+// sorting.
 //
 // The reference joins with a dict and groups the pairs by output coordinate
 // with a second dict and a sort (execution/sparse_dispatch.py:29-82,
@@ -801,7 +802,7 @@ __global__ __launch_bounds__(kRowThreads) void row_fill_kernel(
 // lhs tiles in order and every pair is a segment.  One launch in place of the
 // count and the fill, whose blocks would each take runs of one pair (4,915
 // runs: 41 + 93 us against 9 us).  Block b counts the matches before its
-// tiles itself (kRowMaxLhs tiles at most: 32 lookups a thread, loads in
+// tiles itself (kRowMaxRuns tiles at most: 16 lookups a thread, loads in
 // flight together) and places its own; the last block publishes the counts.
 template <int LN, int RN>
 __global__ __launch_bounds__(kRowThreads) void row_match_kernel(

@@ -33,10 +33,10 @@
 // gives the same bits whether its plan was counted first or queued.
 // Measured (one MI355X), against one thread per output element: block-sparse
 // 6000^2 x dense 6000 x 1500 fp32, 75 x 75 tiles (12,800 pairs, 10.8 GFLOP)
-// 170 us / 3,380 us: 64 TFLOP/s, bound by the fp32 MFMAs (48% busy; the last
-// of 6.25 rounds of workgroups runs half empty).  Sparse x sparse 10240^2
-// bf16, 80 x 80 tiles (5,240 pairs) 32 us / 1,750 us, bound by the latency of
-// one or two K blocks per wave.
+// 170 us / 3,380 us: 64 TFLOP/s, fp32 MFMAs 47% busy (two workgroups fit a CU, so
+// the 1,600 run as three full rounds of 512 and an eighth of a fourth).  Sparse x
+// sparse 10240^2 bf16, 80 x 80 tiles (5,240 pairs) 32 us / 1,750 us, bound by the
+// latency of a pair's three K blocks, the only ones of most segments.
 #pragma once
 
 #include <algorithm>

@@ -432,8 +432,8 @@ def _row_key(lhs, rhs, lc, rc, keys, agg):
 
 
 def _row_step(lhs, rhs, keys, agg, lc, rc, operands, out_dtype, bound, pair_key, events):
-    """The whole step on the sorted row plan (three plan launches, then the
-    fused einsum) when the join's structure suits it: (result, step,
+    """The whole step on the sorted row plan (two or three plan launches, then
+    the fused einsum) when the join's structure suits it: (result, step,
     row hint key), or None.  A pair bound that proves too small is raised to
     the count and the step queued once more; a device-side miss (data not
     sorted, or beyond the plan's counts) is remembered for these coordinate

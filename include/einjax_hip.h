@@ -373,7 +373,8 @@ int ej_dense_plan_async(const int32_t *lhs_coords, int64_t n_lhs, int32_t lhs_nc
                         int32_t *run_order, int32_t *run_order_written, int64_t *dev_counts,
                         int64_t *counts, int32_t counts_direct, ej_stream_t stream);
 
-/* Join and segment plan, in three launches and without sorting, for a join
+/* Join and segment plan, in three launches (two where tile meets tile, as in an
+ * elementwise product) and without sorting, for a join
  * of two sorted sparse relations with the structure of ej_dense_plan_async
  * (no counterpart in the reference, whose join and grouping run on the host,
  * sparse_dispatch.py:29-82, :129-171; the results are the same): the join
